@@ -14,16 +14,26 @@
 //       column potentials v, one Dijkstra-like search per row);
 //   (4) the QCP RMSD of the relabelled selection against the reference; with
 //       superpose, the frame (every atom, centred) is rotated by R1 R2.
-// One wave per frame: the columns of a search are spread over the lanes,
-// the search's minimum is a wave reduction (ties to the lowest column), and
-// the group's reference coordinates, potentials and search state sit in
-// LDS (sized to keep eight waves per CU for groups of a few hundred atoms).
+// Two waves per frame.  Most rows of a group need no search: every row's
+// nearest column is found first, on the matrix cores and by both waves, and
+// rows whose nearest columns differ are matched at once.  The first wave does
+// all else; the columns of a search are spread over its lanes, and the
+// search's minimum is a wave reduction (ties to the lowest column).  The
+// group's reference coordinates, potentials and search state sit in LDS (sized
+// to keep eight frames per CU for groups of a few hundred atoms).
+// What bounds it (20,000 frames x 400 atoms, one group of 300; 8.05 ms a call
+// when every row was searched for, 0.60 ms now): the latency of a frame's
+// serial steps, about 119,000 cycles (gather 17, fit 16, nearest columns 41,
+// two searches of two passes 25, the rest 20 thousand) with eight frames
+// resident per CU.
 #include "common.h"
 
 namespace hr {
 namespace {
 
-constexpr int kLpBlock = kWave;  // one wave per frame
+constexpr int kLpBlock = kWave;
+constexpr int kLpFrameBlock = 2 * kWave;
+constexpr int kLpBatch = 5;  // atoms or columns a lane handles at a time
 constexpr size_t kLpLdsMax = 64 * 1024;
 
 size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
@@ -45,6 +55,16 @@ __device__ __forceinline__ void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Sum of the wave, in every lane: rows of 16 by DPP moves, then two lane
+// exchanges (six exchanges of both halves of a double cost about 800 cycles of
+// latency, and a frame takes some thirty sums).
+__device__ __forceinline__ double lp_sum(double v) {
+    v = row16_sum(v);
+    v += __shfl_xor(v, 16, kWave);
+    v += __shfl_xor(v, 32, kWave);
+    return v;
 }
 
 // Index arrays live on the device, where the host cannot check them: every
@@ -150,7 +170,137 @@ __device__ __forceinline__ void wave_argmin(double& best, int& col) {
                                                 __shfl_xor(col, m, kWave));
 }
 
-__global__ __launch_bounds__(kLpBlock) void lp_frame_kernel(LpArgs A) {
+// euclidean_permutation.cpp: squares of float differences, summed in double
+__device__ __forceinline__ double lp_cost(float dx, float dy, float dz) {
+    return (double)__fmul_rn(dx, dx) + (double)__fmul_rn(dy, dy) + (double)__fmul_rn(dz, dz);
+}
+
+// The two least of two disjoint sets, and the place of the least.
+__device__ __forceinline__ void lp_merge(float& best, float& second, int& arg, float o_best,
+                                         float o_second, int o_arg) {
+    second = fminf(fmaxf(best, o_best), fminf(second, o_second));
+    arg = o_best < best ? o_arg : arg;
+    best = fminf(best, o_best);
+}
+
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+// Start of a group's assignment: u[i] = the least cost of row i (v = 0, so
+// the duals are feasible) and col[i] its column, rows i = 1 .. k.  All k^2
+// pairs are compared once, on the matrix cores: |b|^2 - 2 a.b, the squared
+// distance less the row's own |a|^2, is a product over four terms, two
+// v_mfma_f32_32x32x2_f32 for 32 targets (rows of the tile) by 32 reference
+// atoms (its columns, one per lane of each half wave), and what is left for
+// the vector units is three instructions a pair: the place into the value's
+// last bits, the least and the second least.  (Costing each pair in float
+// there, ten instructions a pair, measured 759 us a call of 20,000 frames with
+// 300 interchangeable atoms; this, 601 us.)  A row whose two least values are
+// further apart than rounding can move them takes the double cost of the
+// nearer target; one that is closer (or not finite) is scanned again in double
+// by the whole wave, ties to the lowest column.  With m the largest |a|^2 or
+// |b|^2 a value (below 3 m) is off by 3 m 2^-19 for its last four bits, by
+// 1.2 m 2^-20 for the product's roundings, and the double cost, of float
+// squares, by m 2^-20: two values by 16.4 m 2^-20 together; tol is twice that.
+// Returns whether every row of the lane has a finite least cost.
+//   q   the group's target atoms as x, z, y, |b|^2, 16-byte aligned
+//   biggest   the largest |b|^2
+//   first   0 or 32: the wave's first row
+__device__ __forceinline__ bool lp_row_minima(const float* q, int k, const float* grx,
+                                              const float* gry, const float* grz, float biggest,
+                                              double* u, int* col, int lane, int first) {
+    bool finite = true;
+    // -inf, unknown to the compiler: as a minimum it would first quiet both
+    // operands, an instruction each
+    float lowest = -__builtin_huge_valf();
+    asm("" : "+v"(lowest));
+    const int half = lane >> 5, in = lane & 31;
+    for (int r0 = first; r0 < k; r0 += 64) {
+        const int r = min(r0 + in, k - 1);
+        const float x = grx[r], y = gry[r], z = grz[r];
+        const float aa = fmaf(x, x, fmaf(y, y, z * z));
+        const float b0 = -2.0f * (half ? y : x), b1 = half ? 1.0f : -2.0f * z;
+        // two tiles at a time: their products and the two chains of least
+        // values overlap
+        float best[2], second[2];
+        int tile[2];
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            best[c] = second[c] = __builtin_huge_valf();
+            tile[c] = 0;
+        }
+        for (int t = 0; t < k; t += 64) {
+            f32x16 d[2] = {};
+            float2 a[2];
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                a[c] = *reinterpret_cast<const float2*>(q + 4 * min(t + 32 * c + in, k - 1) +
+                                                        2 * half);
+                // targets past the group are farther than any
+                if (half && t + 32 * c + in >= k) a[c].y = 1e30f;
+            }
+#pragma unroll
+            for (int c = 0; c < 2; ++c) d[c] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[c].x, b0, d[c], 0, 0, 0);
+#pragma unroll
+            for (int c = 0; c < 2; ++c) d[c] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[c].y, b1, d[c], 0, 0, 0);
+            const float before[2] = {best[0], best[1]};
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+#pragma unroll
+                for (int c = 0; c < 2; ++c) {
+                    // the place in the tile rides in the value's last four bits
+                    const float v = __int_as_float((__float_as_int(d[c][e]) & ~15) | e);
+                    second[c] = __builtin_amdgcn_fmed3f(v, best[c], second[c]);
+                    best[c] = __builtin_amdgcn_fmed3f(v, best[c], lowest);  // the lesser
+                }
+            }
+#pragma unroll
+            for (int c = 0; c < 2; ++c) tile[c] = best[c] < before[c] ? t + 32 * c : tile[c];
+        }
+        int args[2];
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            const int e = __float_as_int(best[c]) & 15;
+            args[c] = tile[c] + 8 * (e / 4) + 4 * half + e % 4;
+        }
+        lp_merge(best[0], second[0], args[0], best[1], second[1], args[1]);
+        // the other half wave's targets of the same row
+        lp_merge(best[0], second[0], args[0], __shfl_xor(best[0], 32, kWave),
+                 __shfl_xor(second[0], 32, kWave), __shfl_xor(args[0], 32, kWave));
+        const bool mine = half == 0 && r0 + in < k;
+        const float* near = q + 4 * min(args[0], k - 1);
+        double least = lp_cost(x - near[0], y - near[2], z - near[1]);
+        const float tol = 0x1p-15f * fmaxf(aa, biggest);
+        // the close rows, one by one, the columns spread over the lanes
+        for (unsigned long long close = __ballot(mine && !(second[0] > best[0] + tol)); close;
+             close &= close - 1) {
+            const int l = __ffsll((long long)close) - 1;
+            const float rx = __shfl(x, l, kWave), ry = __shfl(y, l, kWave), rz = __shfl(z, l, kWave);
+            double c_best = __builtin_huge_val();
+            int c_col = INT_MAX;
+            for (int m = lane; m < k; m += kWave) {
+                const double c = lp_cost(rx - q[4 * m], ry - q[4 * m + 2], rz - q[4 * m + 1]);
+                if (c < c_best) {
+                    c_best = c;
+                    c_col = m;
+                }
+            }
+            wave_argmin(c_best, c_col);
+            if (lane == l) {
+                least = c_best;
+                args[0] = c_col;
+            }
+        }
+        if (mine) {
+            finite = finite && least < __builtin_huge_val();
+            u[r + 1] = least;
+            col[r + 1] = args[0] + 1;
+        }
+    }
+    return finite;
+}
+
+// Two waves a frame: the second only shares the row minima.
+__global__ __launch_bounds__(kLpFrameBlock, 4) void lp_frame_kernel(LpArgs A) {
     extern __shared__ __align__(16) unsigned char lds[];
     const int k1 = A.kmax + 1;
     double* u = reinterpret_cast<double*>(lds);
@@ -167,7 +317,12 @@ __global__ __launch_bounds__(kLpBlock) void lp_frame_kernel(LpArgs A) {
     float* tz = ty + A.n_sel;
     unsigned char* used = reinterpret_cast<unsigned char*>(tz + A.n_sel);
 
-    const int lane = threadIdx.x;
+    const int lane = threadIdx.x & (kWave - 1);
+    const bool lead = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave) == 0;
+    __shared__ int s_finite;
+    __shared__ float s_biggest;
+    __shared__ float s_rot[9];  // R1
+    __shared__ double s_tg;     // the target selection's trace
     const long long f = blockIdx.x;
     float* fr = A.xyz + f * 3LL * A.n_atoms;
     const int n = A.n_sel;
@@ -175,90 +330,102 @@ __global__ __launch_bounds__(kLpBlock) void lp_frame_kernel(LpArgs A) {
     const float* ry = rx + n;
     const float* rz = ry + n;
 
-    // (1) gather and centre the selection
-    double s[3] = {0.0, 0.0, 0.0};
-    for (int a = lane; a < n; a += kWave) {
-        const long long at = clamp_index(A.idx[a], A.n_atoms);
-        const float x = fr[3 * at], y = fr[3 * at + 1], z = fr[3 * at + 2];
-        tx[a] = x;
-        ty[a] = y;
-        tz[a] = z;
-        s[0] += x;
-        s[1] += y;
-        s[2] += z;
-    }
-    double mu[3];
+    double M2[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+    if (lead) {
+        float R1[9] = {1.f, 0.f, 0.f, 0.f, 1.f, 0.f, 0.f, 0.f, 1.f};
+        double tg = 0.0;
+        // (1) gather and centre the selection
+        double s[3] = {0.0, 0.0, 0.0};
+        // loads of kLpBatch atoms a lane at a time, so that their latencies overlap
+        for (int a0 = lane; a0 < n; a0 += kLpBatch * kWave) {
+            long long at[kLpBatch];
+            float x[kLpBatch], y[kLpBatch], z[kLpBatch];
 #pragma unroll
-    for (int c = 0; c < 3; ++c) mu[c] = wave_sum(s[c]) / n;
-    double tg = 0.0;
-    for (int a = lane; a < n; a += kWave) {
-        const float x = (float)((double)tx[a] - mu[0]);
-        const float y = (float)((double)ty[a] - mu[1]);
-        const float z = (float)((double)tz[a] - mu[2]);
-        tx[a] = x;
-        ty[a] = y;
-        tz[a] = z;
-        tg += (double)x * x + (double)y * y + (double)z * z;
-    }
-    tg = wave_sum(tg);
-    __syncthreads();
-
-    // (2) fit on the distinguishable atoms
-    float R1[9] = {1.f, 0.f, 0.f, 0.f, 1.f, 0.f, 0.f, 0.f, 1.f};
-    if (A.n_dis > 0) {
-        const int nd = A.n_dis;
-        double d[3] = {0.0, 0.0, 0.0};
-        for (int k = lane; k < nd; k += kWave) {
-            const int a = clamp_index(A.dis[k], n);
-            d[0] += tx[a];
-            d[1] += ty[a];
-            d[2] += tz[a];
-        }
-        double dm[3];
+            for (int t = 0; t < kLpBatch; ++t)
+                at[t] = 3LL * clamp_index(A.idx[min(a0 + t * kWave, n - 1)], A.n_atoms);
 #pragma unroll
-        for (int c = 0; c < 3; ++c) dm[c] = wave_sum(d[c]) / nd;
-        double M[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0}, ga = 0.0;
-        const float* qx = A.rdis;
-        const float* qy = qx + nd;
-        const float* qz = qy + nd;
-        for (int k = lane; k < nd; k += kWave) {
-            const int a = clamp_index(A.dis[k], n);
-            const double t[3] = {tx[a] - dm[0], ty[a] - dm[1], tz[a] - dm[2]};
-            const double r[3] = {qx[k], qy[k], qz[k]};
+            for (int t = 0; t < kLpBatch; ++t) {
+                x[t] = fr[at[t]];
+                y[t] = fr[at[t] + 1];
+                z[t] = fr[at[t] + 2];
+            }
 #pragma unroll
-            for (int i = 0; i < 3; ++i) {
-#pragma unroll
-                for (int j = 0; j < 3; ++j) M[3 * i + j] = fma(t[i], r[j], M[3 * i + j]);
-                ga = fma(t[i], t[i], ga);
+            for (int t = 0; t < kLpBatch; ++t) {
+                const int a = a0 + t * kWave;
+                if (a < n) {
+                    tx[a] = x[t];
+                    ty[a] = y[t];
+                    tz[a] = z[t];
+                    s[0] += x[t];
+                    s[1] += y[t];
+                    s[2] += z[t];
+                }
             }
         }
+        double mu[3];
 #pragma unroll
-        for (int e = 0; e < 9; ++e) M[e] = wave_sum(M[e]);
-        ga = wave_sum(ga);
-        double R[9];
-        qcp_solve<true>(M, 0.5 * (ga + A.traces[1]), R);
-#pragma unroll
-        for (int e = 0; e < 9; ++e) R1[e] = (float)R[e];
+        for (int c = 0; c < 3; ++c) mu[c] = lp_sum(s[c]) / n;
         for (int a = lane; a < n; a += kWave) {
-            const float x = tx[a], y = ty[a], z = tz[a];
-            tx[a] = x * R1[0] + y * R1[3] + z * R1[6];
-            ty[a] = x * R1[1] + y * R1[4] + z * R1[7];
-            tz[a] = x * R1[2] + y * R1[5] + z * R1[8];
+            const float x = (float)((double)tx[a] - mu[0]);
+            const float y = (float)((double)ty[a] - mu[1]);
+            const float z = (float)((double)tz[a] - mu[2]);
+            tx[a] = x;
+            ty[a] = y;
+            tz[a] = z;
+            tg += (double)x * x + (double)y * y + (double)z * z;
         }
-        __syncthreads();
-    }
+        tg = lp_sum(tg);
+        wave_sync();
 
-    // correlation of the relabelled selection with the reference: the
-    // distinguishable atoms keep their labels
-    double M2[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-    for (int k = lane; k < A.n_dis; k += kWave) {
-        const int a = clamp_index(A.dis[k], n);
-        const double t[3] = {tx[a], ty[a], tz[a]};
-        const double r[3] = {rx[a], ry[a], rz[a]};
+        // (2) fit on the distinguishable atoms
+        if (A.n_dis > 0) {
+            const int nd = A.n_dis;
+            double d[3] = {0.0, 0.0, 0.0};
+            for (int k = lane; k < nd; k += kWave) {
+                const int a = clamp_index(A.dis[k], n);
+                d[0] += tx[a];
+                d[1] += ty[a];
+                d[2] += tz[a];
+            }
+            double dm[3];
 #pragma unroll
-        for (int i = 0; i < 3; ++i)
+            for (int c = 0; c < 3; ++c) dm[c] = lp_sum(d[c]) / nd;
+            double M[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0}, ga = 0.0;
+            const float* qx = A.rdis;
+            const float* qy = qx + nd;
+            const float* qz = qy + nd;
+            for (int k = lane; k < nd; k += kWave) {
+                const int a = clamp_index(A.dis[k], n);
+                const double t[3] = {tx[a] - dm[0], ty[a] - dm[1], tz[a] - dm[2]};
+                const double r[3] = {qx[k], qy[k], qz[k]};
 #pragma unroll
-            for (int j = 0; j < 3; ++j) M2[3 * i + j] = fma(t[i], r[j], M2[3 * i + j]);
+                for (int i = 0; i < 3; ++i) {
+#pragma unroll
+                    for (int j = 0; j < 3; ++j) M[3 * i + j] = fma(t[i], r[j], M[3 * i + j]);
+                    ga = fma(t[i], t[i], ga);
+                }
+            }
+#pragma unroll
+            for (int e = 0; e < 9; ++e) M[e] = lp_sum(M[e]);
+            ga = lp_sum(ga);
+            double R[9];
+            qcp_solve<true>(M, 0.5 * (ga + A.traces[1]), R);
+#pragma unroll
+            for (int e = 0; e < 9; ++e) R1[e] = (float)R[e];
+            for (int a = lane; a < n; a += kWave) {
+                const float x = tx[a], y = ty[a], z = tz[a];
+                tx[a] = x * R1[0] + y * R1[3] + z * R1[6];
+                ty[a] = x * R1[1] + y * R1[4] + z * R1[7];
+                tz[a] = x * R1[2] + y * R1[5] + z * R1[8];
+            }
+            wave_sync();
+        }
+
+        if (lane == 0) {
+            s_tg = tg;
+#pragma unroll
+            for (int e = 0; e < 9; ++e) s_rot[e] = R1[e];
+        }
     }
 
     // (3) the assignment inside each group
@@ -267,84 +434,171 @@ __global__ __launch_bounds__(kLpBlock) void lp_frame_kernel(LpArgs A) {
         const int k = A.group_off[g + 1] - g0;
         if (k <= 0) continue;
         if (k > A.kmax) {  // larger than the LDS was sized for: no result
-            if (lane == 0) A.out[f] = __builtin_nanf("");
+            if (lead && lane == 0) A.out[f] = __builtin_nanf("");
             return;
         }
-        for (int j = lane; j < k; j += kWave) {
-            const int a = clamp_index(A.group_atoms[g0 + j], n);
-            gat[j] = a;
-            grx[j] = rx[a];
-            gry[j] = ry[a];
-            grz[j] = rz[a];
+        float* q = reinterpret_cast<float*>(minv);
+        int* col = reinterpret_cast<int*>(v);
+        // the group's target atoms where minv, p and way will be (16 k1 bytes,
+        // after two arrays of 8 k1), the rows' columns where v will be
+        if (lead) {
+            float biggest = 0.0f;
+            for (int b0 = lane; b0 < k; b0 += kLpBatch * kWave) {
+                int at[kLpBatch];
+                float x[kLpBatch], y[kLpBatch], z[kLpBatch];
+#pragma unroll
+                for (int t = 0; t < kLpBatch; ++t)
+                    at[t] = clamp_index(A.group_atoms[g0 + min(b0 + t * kWave, k - 1)], n);
+#pragma unroll
+                for (int t = 0; t < kLpBatch; ++t) {
+                    x[t] = rx[at[t]];
+                    y[t] = ry[at[t]];
+                    z[t] = rz[at[t]];
+                }
+#pragma unroll
+                for (int t = 0; t < kLpBatch; ++t) {
+                    const int j = b0 + t * kWave, a = at[t];
+                    if (j < k) {
+                        const float bb = fmaf(tx[a], tx[a], fmaf(ty[a], ty[a], tz[a] * tz[a]));
+                        *reinterpret_cast<float4*>(q + 4 * j) = make_float4(tx[a], tz[a], ty[a], bb);
+                        biggest = fmaxf(biggest, bb);
+                        gat[j] = a;
+                        grx[j] = x[t];
+                        gry[j] = y[t];
+                        grz[j] = z[t];
+                    }
+                }
+            }
+#pragma unroll
+            for (int m = 1; m < kWave; m <<= 1) biggest = fmaxf(biggest, __shfl_xor(biggest, m, kWave));
+            if (lane == 0) {
+                s_finite = 1;
+                s_biggest = biggest;
+            }
         }
+        __syncthreads();
+        // Greedy start: every row's least cost as its dual, and the row itself
+        // in that column unless a lower row is there.  Rows left over (two
+        // reference atoms nearest to one target atom) are searched for; from
+        // empty duals every row was (8.0 ms a call of 20,000 frames x 300
+        // interchangeable atoms).
+        if (!lp_row_minima(q, k, grx, gry, grz, s_biggest, u, col, lane, lead ? 0 : 32)) s_finite = 0;
+        __syncthreads();
+        if (!lead) continue;
+        const bool greedy = s_finite != 0;
         for (int j = lane; j <= k; j += kWave) {
-            u[j] = 0.0;
-            v[j] = 0.0;
-            p[j] = 0;
+            p[j] = greedy ? INT_MAX : 0;
+            way[j] = j ? col[j] : 0;
+            if (!greedy || j == 0) u[j] = 0.0;
+        }
+        wave_sync();
+        for (int j = lane; j <= k; j += kWave) v[j] = 0.0;
+        if (greedy)
+            for (int i = 1 + lane; i <= k; i += kWave) atomicMin(&p[way[i]], i);
+        wave_sync();
+        unsigned free_rows = 0;  // bit s: row 1 + lane + 64 s has no column
+        for (int s = 0; s * kWave < k; ++s) {
+            const int i = 1 + lane + s * kWave;
+            if (i <= k && !(greedy && p[way[i]] == i)) free_rows |= 1u << s;
+        }
+        wave_sync();
+        for (int j = lane; j <= k; j += kWave) {
+            if (p[j] == INT_MAX) p[j] = 0;
             way[j] = 0;
         }
         wave_sync();
-        for (int i = 1; i <= k; ++i) {
-            for (int j = lane; j <= k; j += kWave) {
-                minv[j] = __builtin_huge_val();
-                used[j] = 0;
-            }
-            if (lane == 0) p[0] = i;
-            wave_sync();
-            int j0 = 0;
-            // each pass marks one more column used; a free column (p = 0) is
-            // reached within i passes, so the loop ends for any costs
-            for (int pass = 0; pass <= k; ++pass) {
-                if (lane == 0) used[j0] = 1;
-                wave_sync();
-                const int i0 = p[j0];
-                const float qx = grx[i0 - 1], qy = gry[i0 - 1], qz = grz[i0 - 1];
-                const double ui = u[i0];
-                double best = __builtin_huge_val();
-                int col = INT_MAX;
-                for (int j = 1 + lane; j <= k; j += kWave) {
-                    if (used[j]) continue;
-                    // euclidean_permutation.cpp: squares of float differences, summed in double
-                    const int ta = gat[j - 1];
-                    const float dx = qx - tx[ta], dy = qy - ty[ta], dz = qz - tz[ta];
-                    const double c = (double)__fmul_rn(dx, dx) + (double)__fmul_rn(dy, dy) +
-                                     (double)__fmul_rn(dz, dz);
-                    const double cur = c - ui - v[j];
-                    double mv = minv[j];
-                    if (cur < mv) {
-                        mv = cur;
-                        minv[j] = cur;
-                        way[j] = j0;
-                    }
-                    if (mv < best || col == INT_MAX) {
-                        best = mv;
-                        col = j;
-                    }
-                }
-                wave_argmin(best, col);
-                const double delta = best;
-                wave_sync();  // every lane has read u[i0] before it changes
+        for (int s = 0; s * kWave < k; ++s) {
+            for (unsigned long long rows = __ballot((free_rows >> s) & 1u); rows; rows &= rows - 1) {
+                const int i = s * kWave + __ffsll((long long)rows);
                 for (int j = lane; j <= k; j += kWave) {
-                    if (used[j]) {
-                        u[p[j]] += delta;
-                        v[j] -= delta;
-                    } else {
-                        minv[j] -= delta;
+                    minv[j] = __builtin_huge_val();
+                    used[j] = 0;
+                }
+                if (lane == 0) p[0] = i;
+                wave_sync();
+                int j0 = 0;
+                // each pass marks one more column used; a free column (p = 0) is
+                // reached within i passes, so the loop ends for any costs
+                for (int pass = 0; pass <= k; ++pass) {
+                    if (lane == 0) used[j0] = 1;
+                    wave_sync();
+                    const int i0 = p[j0];
+                    const float qx = grx[i0 - 1], qy = gry[i0 - 1], qz = grz[i0 - 1];
+                    const double ui = u[i0];
+                    double best = __builtin_huge_val();
+                    int at = INT_MAX;
+                    for (int b0 = 1 + lane; b0 <= k; b0 += kLpBatch * kWave) {
+                        bool open[kLpBatch];
+                        int ta[kLpBatch];
+                        double vj[kLpBatch], mv[kLpBatch];
+                        float dx[kLpBatch], dy[kLpBatch], dz[kLpBatch];
+#pragma unroll
+                        for (int t = 0; t < kLpBatch; ++t) {
+                            const int j = min(b0 + t * kWave, k);
+                            open[t] = b0 + t * kWave <= k && !used[j];
+                            ta[t] = gat[j - 1];
+                            vj[t] = v[j];
+                            mv[t] = minv[j];
+                        }
+#pragma unroll
+                        for (int t = 0; t < kLpBatch; ++t) {
+                            dx[t] = qx - tx[ta[t]];
+                            dy[t] = qy - ty[ta[t]];
+                            dz[t] = qz - tz[ta[t]];
+                        }
+#pragma unroll
+                        for (int t = 0; t < kLpBatch; ++t) {
+                            const int j = b0 + t * kWave;
+                            const double cur = lp_cost(dx[t], dy[t], dz[t]) - ui - vj[t];
+                            if (open[t]) {
+                                if (cur < mv[t]) {
+                                    mv[t] = cur;
+                                    minv[j] = cur;
+                                    way[j] = j0;
+                                }
+                                if (mv[t] < best || at == INT_MAX) {
+                                    best = mv[t];
+                                    at = j;
+                                }
+                            }
+                        }
+                    }
+                    wave_argmin(best, at);
+                    const double delta = best;
+                    wave_sync();  // every lane has read u[i0] before it changes
+                    for (int b0 = lane; b0 <= k; b0 += kLpBatch * kWave) {
+                        bool taken[kLpBatch];
+                        double was[kLpBatch];
+#pragma unroll
+                        for (int t = 0; t < kLpBatch; ++t) taken[t] = used[min(b0 + t * kWave, k)];
+#pragma unroll
+                        for (int t = 0; t < kLpBatch; ++t) {
+                            const int j = min(b0 + t * kWave, k);
+                            was[t] = taken[t] ? v[j] : minv[j];
+                        }
+#pragma unroll
+                        for (int t = 0; t < kLpBatch; ++t) {
+                            const int j = b0 + t * kWave;
+                            if (j <= k) {
+                                if (taken[t]) u[p[j]] += delta;
+                                (taken[t] ? v : minv)[j] = was[t] - delta;
+                            }
+                        }
+                    }
+                    wave_sync();
+                    j0 = at;
+                    if (p[j0] == 0) break;
+                }
+                if (lane == 0) {
+                    int jj = j0;
+                    for (int step = 0; step <= k && jj != 0; ++step) {
+                        const int j1 = way[jj];
+                        p[jj] = p[j1];
+                        jj = j1;
                     }
                 }
                 wave_sync();
-                j0 = col;
-                if (p[j0] == 0) break;
             }
-            if (lane == 0) {
-                int jj = j0;
-                for (int step = 0; step <= k && jj != 0; ++step) {
-                    const int j1 = way[jj];
-                    p[jj] = p[j1];
-                    jj = j1;
-                }
-            }
-            wave_sync();
         }
         // column j (target atom gat[j - 1]) takes row p[j] (reference atom gat[p[j] - 1])
         for (int j = 1 + lane; j <= k; j += kWave) {
@@ -358,11 +612,24 @@ __global__ __launch_bounds__(kLpBlock) void lp_frame_kernel(LpArgs A) {
         }
         wave_sync();  // the next group overwrites the group's arrays
     }
+    if (!lead) return;
+
+    // correlation of the relabelled selection with the reference: the
+    // distinguishable atoms keep their labels
+    for (int k = lane; k < A.n_dis; k += kWave) {
+        const int a = clamp_index(A.dis[k], n);
+        const double t[3] = {tx[a], ty[a], tz[a]};
+        const double r[3] = {rx[a], ry[a], rz[a]};
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+#pragma unroll
+            for (int j = 0; j < 3; ++j) M2[3 * i + j] = fma(t[i], r[j], M2[3 * i + j]);
+    }
 
     // (4) QCP on the relabelled selection
 #pragma unroll
-    for (int e = 0; e < 9; ++e) M2[e] = wave_sum(M2[e]);
-    const double rg = A.traces[0];
+    for (int e = 0; e < 9; ++e) M2[e] = lp_sum(M2[e]);
+    const double rg = A.traces[0], tg = s_tg;
     double R2[9];
     double lam;
     if (A.superpose)
@@ -381,7 +648,7 @@ __global__ __launch_bounds__(kLpBlock) void lp_frame_kernel(LpArgs A) {
         for (int j = 0; j < 3; ++j) {
             float acc = 0.f;
 #pragma unroll
-            for (int q = 0; q < 3; ++q) acc += R1[3 * i + q] * (float)R2[3 * q + j];
+            for (int q = 0; q < 3; ++q) acc += s_rot[3 * i + q] * (float)R2[3 * q + j];
             R3[3 * i + j] = acc;
         }
     double w[3] = {0.0, 0.0, 0.0};
@@ -392,7 +659,7 @@ __global__ __launch_bounds__(kLpBlock) void lp_frame_kernel(LpArgs A) {
     }
     double wm[3];
 #pragma unroll
-    for (int c = 0; c < 3; ++c) wm[c] = wave_sum(w[c]) / A.n_atoms;
+    for (int c = 0; c < 3; ++c) wm[c] = lp_sum(w[c]) / A.n_atoms;
     for (int a = lane; a < A.n_atoms; a += kWave) {
         const float x = (float)((double)fr[3LL * a] - wm[0]);
         const float y = (float)((double)fr[3LL * a + 1] - wm[1]);
@@ -464,7 +731,12 @@ int hr_lprmsd(float* xyz, int64_t n_frames, int32_t n_atoms, const float* ref_fr
     A.traces = traces;
     A.superpose = superpose ? 1 : 0;
     A.out = out;
-    hipLaunchKernelGGL(lp_frame_kernel, dim3((unsigned)n_frames), dim3(kLpBlock), lds, s, A);
+    // the kernel's own few words count towards the default limit of 64 KiB too
+    if (lds > kLpLdsMax - 256)
+        HR_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(lp_frame_kernel),
+                                         hipFuncAttributeMaxDynamicSharedMemorySize,
+                                         (int)kLpLdsMax));
+    hipLaunchKernelGGL(lp_frame_kernel, dim3((unsigned)n_frames), dim3(kLpFrameBlock), lds, s, A);
     return launch_status("lp_frame_kernel");
 }
 
