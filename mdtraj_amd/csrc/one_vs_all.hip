@@ -7,6 +7,8 @@
 // solve then runs one lane per frame (lane k finishes the k-th frame of the
 // wave's current group of 64).  The reference selection and the atom indices
 // are staged once per workgroup in LDS.
+#include <limits.h>
+
 #include <algorithm>
 
 #include "frames.h"
@@ -140,35 +142,254 @@ __global__ __launch_bounds__(kBlock) void center_kernel(float* __restrict__ xyz,
     }
 }
 
-// x' = float(float(x - mu_f) R + mu_ref) over every atom of every frame,
-// rounding as Trajectory.superpose does (float64 offsets applied to float32
-// coordinates, float32 rotation, core/trajectory.py:1135-1171).
+// x' = float(float(x - mu_f) R + mu_ref) of one atom, rounding as
+// Trajectory.superpose does (float64 offsets applied to float32 coordinates,
+// float32 rotation, core/trajectory.py:1135-1171); without translate x' = x R.
+__device__ __forceinline__ void move_atom(float ax, float ay, float az, const float (&R)[9],
+                                          const double (&m)[3], const double (&to)[3],
+                                          int translate, float (&o)[3]) {
+    const float x = translate ? (float)((double)ax - m[0]) : ax;
+    const float y = translate ? (float)((double)ay - m[1]) : ay;
+    const float z = translate ? (float)((double)az - m[2]) : az;
+    const float tx = x * R[0] + y * R[3] + z * R[6];
+    const float ty = x * R[1] + y * R[4] + z * R[7];
+    const float tz = x * R[2] + y * R[5] + z * R[8];
+    o[0] = translate ? (float)((double)tx + to[0]) : tx;
+    o[1] = translate ? (float)((double)ty + to[1]) : ty;
+    o[2] = translate ? (float)((double)tz + to[2]) : tz;
+}
+
+// Every atom of every frame moved by its frame's fit.
 __global__ __launch_bounds__(kBlock) void apply_kernel(float* __restrict__ xyz, long long n_frames,
                                                        int n_atoms, const float* __restrict__ rot,
                                                        const double* __restrict__ mu,
                                                        const double* __restrict__ ref_stats,
                                                        double n_ref, int translate) {
-    const double rmx = translate ? ref_stats[0] / n_ref : 0.0;
-    const double rmy = translate ? ref_stats[1] / n_ref : 0.0;
-    const double rmz = translate ? ref_stats[2] / n_ref : 0.0;
+    double to[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+    for (int c = 0; c < 3; ++c) to[c] = translate ? ref_stats[c] / n_ref : 0.0;
     for (long long f = blockIdx.x; f < n_frames; f += gridDim.x) {
         float R[9];
 #pragma unroll
         for (int i = 0; i < 9; ++i) R[i] = rot[9 * f + i];
-        const double mx = translate ? mu[3 * f] : 0.0;
-        const double my = translate ? mu[3 * f + 1] : 0.0;
-        const double mz = translate ? mu[3 * f + 2] : 0.0;
+        double m[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+        for (int c = 0; c < 3; ++c) m[c] = translate ? mu[3 * f + c] : 0.0;
         float* fr = xyz + f * 3LL * n_atoms;
         for (int a = threadIdx.x; a < n_atoms; a += kBlock) {
-            const float x = translate ? (float)((double)fr[3 * a] - mx) : fr[3 * a];
-            const float y = translate ? (float)((double)fr[3 * a + 1] - my) : fr[3 * a + 1];
-            const float z = translate ? (float)((double)fr[3 * a + 2] - mz) : fr[3 * a + 2];
-            const float tx = x * R[0] + y * R[3] + z * R[6];
-            const float ty = x * R[1] + y * R[4] + z * R[7];
-            const float tz = x * R[2] + y * R[5] + z * R[8];
-            fr[3 * a] = translate ? (float)((double)tx + rmx) : tx;
-            fr[3 * a + 1] = translate ? (float)((double)ty + rmy) : ty;
-            fr[3 * a + 2] = translate ? (float)((double)tz + rmz) : tz;
+            float o[3];
+            move_atom(fr[3 * a], fr[3 * a + 1], fr[3 * a + 2], R, m, to, translate, o);
+            fr[3 * a] = o[0];
+            fr[3 * a + 1] = o[1];
+            fr[3 * a + 2] = o[2];
+        }
+    }
+}
+
+// Superposition in one pass over memory: a workgroup holds a run of whole
+// frames in LDS (consecutive in memory), fits every one of them there, and
+// writes the moved atoms back; fitting and moving in two kernels reads the
+// frames twice.
+//   load   16 bytes a lane, kLoads of them in flight
+//   sums   a row of kRL lanes per frame, or kWavesPer waves when a run has
+//          fewer frames than the workgroup has waves (their parts are added
+//          below)
+//   fit    one lane per frame, from the frame's sums in LDS
+//   move   atom by atom to memory; whole waves per frame when frames are
+//          long (the fit stays in registers), else atoms dealt out flat
+// Rounding is the two kernels': the sums are FP64 in another order.
+//
+// Bound by HBM (a read and a write of every atom) as far as four workgroups of
+// a CU, at different steps, keep it busy: 20,000 frames of 3,001 atoms (375 of
+// them fitted), 1.44 GB, in 366 us (3.9 TB/s) against 390 us for two kernels,
+// which move 2.3 GB.  (Two persistent workgroups a CU, each with a second
+// buffer filled by direct loads to LDS, were slower, 417 us: two frames at
+// work on a CU instead of four.  The sums' indices and reference atoms are
+// asked for ahead of the frames; read where they were used, 398 us.)
+constexpr int kLoads = 10;
+// Frames of this many atoms on keep a frame's fit in registers while whole
+// waves move its atoms.
+constexpr int kFlatAtoms = 192;
+
+// Bytes before the coordinates in LDS: per frame the parts' sums, the centroid
+// and the rotation.
+__host__ __device__ __forceinline__ size_t superpose_head(int per_group, int parts) {
+    return ((size_t)per_group * (parts * 13 * 8 + 3 * 8 + 9 * 4) + 15) / 16 * 16;
+}
+
+template <int kRL, int kWavesPer, bool kGather>
+__global__ __launch_bounds__(kBlock, 4) void superpose_kernel(
+    float* __restrict__ xyz, long long n_frames, int n_atoms, int per_group,
+    const int* __restrict__ idx, int n_sel, const float* __restrict__ ref_sel,
+    const double* __restrict__ ref_stats, int translate, float* __restrict__ rot_out,
+    float* __restrict__ rmsd_out) {
+    typedef float V4f __attribute__((ext_vector_type(4), aligned(4)));
+    static_assert(kWavesPer == 1 || kRL == kWave, "waves share frames as whole rows");
+    constexpr int kThreads = kBlock;
+    constexpr int kNS = SumsPerFrame<Kind::Fit>::value;
+    extern __shared__ __align__(16) unsigned char s_mem[];
+    const int words = 3 * n_atoms;
+    double* s_sum = reinterpret_cast<double*>(s_mem);            // per_group x kWavesPer x kNS
+    double* s_mu = s_sum + (size_t)per_group * kWavesPer * kNS;     // per_group x 3
+    float* s_rot = reinterpret_cast<float*>(s_mu + 3 * per_group);  // per_group x 9
+    float* s_x = reinterpret_cast<float*>(s_mem + superpose_head(per_group, kWavesPer));
+    const int tid = threadIdx.x, lane = tid & (kWave - 1);
+    const int wv = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const long long f0 = (long long)blockIdx.x * per_group;
+    const int cnt = (int)min((long long)per_group, n_frames - f0);
+    float* run = xyz + f0 * words;
+    const int n_words = cnt * words;
+
+    constexpr int kLanes = kWavesPer > 1 ? kWavesPer * kWave : kRL;
+    constexpr int kRows = kThreads / kLanes;
+    const int row = tid / kLanes, t = tid % kLanes;
+    // kItemAtoms atoms of the selection a lane: where they are in a frame and
+    // the reference's
+    struct Item {
+        int at[kItemAtoms];
+        float x[kItemAtoms], y[kItemAtoms], z[kItemAtoms];
+    } a_item, b_item;
+    auto fetch = [&](int item, Item& it) {
+#pragma unroll
+        for (int u = 0; u < kItemAtoms; ++u) {
+            const int j = min(t + (item * kItemAtoms + u) * kLanes, n_sel - 1);
+            it.at[u] = 3 * (kGather ? idx[j] : j);
+            it.x[u] = ref_sel[j];
+            it.y[u] = ref_sel[n_sel + j];
+            it.z[u] = ref_sel[2 * n_sel + j];
+        }
+    };
+    fetch(0, a_item);
+
+    for (int i0 = 4 * tid; i0 < n_words; i0 += 4 * kLoads * kThreads) {
+        V4f v[kLoads];
+#pragma unroll
+        for (int t = 0; t < kLoads; ++t) {
+            // past the run's end: its last 16 bytes again (a run has at least
+            // four words unless it is one atom)
+            const int i = min(i0 + 4 * t * kThreads, max(n_words - 4, 0));
+            if (n_words >= 4) v[t] = *reinterpret_cast<const V4f*>(run + i);
+        }
+#pragma unroll
+        for (int t = 0; t < kLoads; ++t) {
+            const int i = i0 + 4 * t * kThreads;
+            if (i + 4 <= n_words) {
+                *reinterpret_cast<float4*>(s_x + i) = make_float4(v[t].x, v[t].y, v[t].z, v[t].w);
+            } else if (i < n_words) {
+                for (int k = i; k < n_words; ++k) s_x[k] = run[k];
+            }
+        }
+    }
+    __syncthreads();
+
+    // the row's items in turn: frame after frame, item after item; while one is
+    // accumulated the next one's indices and reference atoms are on their way
+    {
+        const int items = (n_sel + kItemAtoms * kLanes - 1) / (kItemAtoms * kLanes);
+        int k = row, item = 0;
+        Sums s = {};
+        auto step = [&](Item& now, Item& next) {
+            const int item_next = item + 1 < items ? item + 1 : 0;
+            fetch(item_next, next);
+            const float* fr = s_x + (k < cnt ? k : 0) * words;
+            float bx[kItemAtoms], by[kItemAtoms], bz[kItemAtoms];
+#pragma unroll
+            for (int u = 0; u < kItemAtoms; ++u) {
+                bx[u] = fr[now.at[u]];
+                by[u] = fr[now.at[u] + 1];
+                bz[u] = fr[now.at[u] + 2];
+            }
+#pragma unroll
+            for (int u = 0; u < kItemAtoms; ++u) {
+                const bool ok = t + (item * kItemAtoms + u) * kLanes < n_sel;
+                accumulate<Kind::Fit>(s, valid_atom(ok, bx[u]), valid_atom(ok, by[u]),
+                                      valid_atom(ok, bz[u]), now.x[u], now.y[u], now.z[u]);
+            }
+            if (item_next == 0) {
+                row_reduce<Kind::Fit, kRL>(s);
+                if (t % kRL == 0 && k < cnt)
+                    store_sums<Kind::Fit>(s_sum + ((size_t)k * kWavesPer + t / kRL) * kNS, s);
+                s = Sums{};
+                k += kRows;
+            }
+            item = item_next;
+        };
+        const int total = (cnt + kRows - 1) / kRows * items;
+        for (int i = 0; i < total; i += 2) {
+            step(a_item, b_item);
+            if (i + 1 < total) step(b_item, a_item);
+        }
+    }
+    __syncthreads();
+
+    const double n = (double)n_sel;
+    if (tid < cnt) {
+        Sums mine;
+        load_sums<Kind::Fit>(mine, s_sum + (size_t)tid * kWavesPer * kNS);
+#pragma unroll
+        for (int w = 1; w < kWavesPer; ++w) {
+            Sums part;
+            load_sums<Kind::Fit>(part, s_sum + ((size_t)tid * kWavesPer + w) * kNS);
+            mine.q += part.q;
+            mine.sx += part.sx;
+            mine.sy += part.sy;
+            mine.sz += part.sz;
+#pragma unroll
+            for (int e = 0; e < 9; ++e) mine.p[e] += part.p[e];
+        }
+        const double rs[4] = {ref_stats[0], ref_stats[1], ref_stats[2], ref_stats[3]};
+        double M[9], ga, gb, R[9];
+        centred(mine, rs, n, M, ga, gb);
+        const double lam = qcp_solve<true>(M, 0.5 * (ga + gb), R);
+        const long long f = f0 + tid;
+#pragma unroll
+        for (int e = 0; e < 9; ++e) {
+            s_rot[9 * tid + e] = (float)R[e];
+            if (rot_out) rot_out[9 * f + e] = (float)R[e];
+        }
+        s_mu[3 * tid] = mine.sx / n;
+        s_mu[3 * tid + 1] = mine.sy / n;
+        s_mu[3 * tid + 2] = mine.sz / n;
+        if (rmsd_out) {
+            const double msd = (ga + gb - 2.0 * lam) / n;
+            rmsd_out[f] = (float)sqrt(msd > 0.0 ? msd : 0.0);
+        }
+    }
+    __syncthreads();
+
+    double to[3];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) to[c] = translate ? ref_stats[c] / n : 0.0;
+    float R[9], o[3];
+    double m[3];
+    auto fit_of = [&](int k) {
+#pragma unroll
+        for (int e = 0; e < 9; ++e) R[e] = s_rot[9 * k + e];
+#pragma unroll
+        for (int c = 0; c < 3; ++c) m[c] = s_mu[3 * k + c];
+    };
+    if (n_atoms >= kFlatAtoms) {
+        constexpr int kStep = kWavesPerBlock / kWavesPer;  // frames side by side
+        for (int k = wv / kWavesPer; k < cnt; k += kStep) {
+            fit_of(k);
+            const float* fr = s_x + k * words;
+            float* dst = run + k * words;
+            for (int a = wv % kWavesPer * kWave + lane; a < n_atoms; a += kWavesPer * kWave) {
+                move_atom(fr[3 * a], fr[3 * a + 1], fr[3 * a + 2], R, m, to, translate, o);
+                dst[3 * a] = o[0];
+                dst[3 * a + 1] = o[1];
+                dst[3 * a + 2] = o[2];
+            }
+        }
+    } else {
+        // frame of atom e: e / n_atoms, exact for e < 2^16 and n_atoms < 2^16
+        const unsigned magic = n_atoms > 1 ? 0xFFFFFFFFu / (unsigned)n_atoms + 1u : 0u;
+        for (int e = tid; e < cnt * n_atoms; e += kThreads) {
+            fit_of(n_atoms > 1 ? (int)__umulhi((unsigned)e, magic) : e);
+            move_atom(s_x[3 * e], s_x[3 * e + 1], s_x[3 * e + 2], R, m, to, translate, o);
+            run[3 * e] = o[0];
+            run[3 * e + 1] = o[1];
+            run[3 * e + 2] = o[2];
         }
     }
 }
@@ -314,6 +535,69 @@ int one_vs_all_fused_ref(hipStream_t s, const float* frames, long long n_frames,
 }
 
 namespace {
+
+// LDS of superpose_kernel for per_group frames.
+size_t superpose_lds(int per_group, int parts, int n_atoms) {
+    return superpose_head(per_group, parts) + 12 * (size_t)per_group * n_atoms;
+}
+
+template <int kRL, int kWavesPer, bool kGather>
+int launch_superpose_v(hipStream_t s, float* xyz, long long n_frames, int n_atoms, int per_group,
+                       const int* idx, int n_sel, const float* ref_sel, const double* stats,
+                       int translate, float* rot_out, float* rmsd_out) {
+    const long long blocks = (n_frames + per_group - 1) / per_group;
+    hipLaunchKernelGGL((superpose_kernel<kRL, kWavesPer, kGather>), dim3((unsigned)blocks),
+                       dim3(kBlock), superpose_lds(per_group, kWavesPer, n_atoms), s, xyz,
+                       n_frames, n_atoms, per_group, idx, n_sel, ref_sel, stats, translate,
+                       rot_out, rmsd_out);
+    return launch_status("superpose_kernel");
+}
+
+// One-pass superposition where it is the faster one; *done is false, and
+// nothing is launched, where the two-kernel path is to be used.
+int superpose_one_pass(hipStream_t s, float* xyz, long long n_frames, int n_atoms, const int* idx,
+                       int n_sel, const float* ref_sel, const double* stats, int translate,
+                       float* rot_out, float* rmsd_out, bool* done) {
+    *done = false;
+    constexpr size_t kLds = 40 * 1000;  // four workgroups a CU
+    auto fits = [&](int group, int waves) { return superpose_lds(group, waves, n_atoms) <= kLds; };
+    int group = 1, waves = 4;
+    if (fits(8, 1)) {
+        group = 8;
+        while (group < kBlock && fits(group + 1, 1)) ++group;
+        waves = 1;
+    } else if (fits(3, 1)) {
+        group = fits(4, 1) ? 4 : 3;
+        waves = 1;
+    } else if (fits(2, 2)) {
+        group = 2;
+        waves = 2;
+    }
+    // Runs that leave much of their LDS empty keep too few bytes on the way, and
+    // the two kernels are the faster ones (us, one pass against two, 1.44 GB:
+    // 420 atoms, 20 KB runs 511 / 462; 1,000 atoms, 36 KB 396 / 415; 1,700,
+    // 20 KB 512 / 436; 2,000, 24 KB 467 / 413; 2,700, 32 KB 406 / 420; 3,001,
+    // 36 KB 366 / 390); so are they for frames that do not fit at all.  Runs of
+    // many short frames always pay, as apply_kernel takes a workgroup per frame:
+    // 8 atoms 704 / 3,303, 22 atoms 522 / 1,470, 100 atoms 414 / 575, 300 atoms
+    // 409 / 497, 400 atoms 415 / 447.
+    const bool full = group >= 8 || 12LL * group * n_atoms >= 32000;
+    if (!full || !fits(group, waves) || (n_frames + group - 1) / group > INT_MAX) return HR_OK;
+    const int rl = n_sel < 28 ? 4 : n_sel < 112 ? 8 : n_sel < 360 ? 16 : 64;
+    *done = true;
+#define HR_SUP(RL, W)                                                                           \
+    (idx ? launch_superpose_v<RL, W, true>(s, xyz, n_frames, n_atoms, group, idx, n_sel,        \
+                                           ref_sel, stats, translate, rot_out, rmsd_out)        \
+         : launch_superpose_v<RL, W, false>(s, xyz, n_frames, n_atoms, group, idx, n_sel,       \
+                                            ref_sel, stats, translate, rot_out, rmsd_out))
+    if (waves == 4) return HR_SUP(kWave, 4);
+    if (waves == 2) return HR_SUP(kWave, 2);
+    return rl == 64   ? HR_SUP(64, 1)
+           : rl == 16 ? HR_SUP(16, 1)
+           : rl == 8  ? HR_SUP(8, 1)
+                      : HR_SUP(4, 1);
+#undef HR_SUP
+}
 
 int prep_ref(hipStream_t s, const float* ref, const int* ref_idx, int n_sel, int axis_rowstride,
              void* workspace, float** ref_sel, double** stats) {
@@ -699,6 +983,12 @@ int hr_superpose(float* xyz, int64_t n_frames, int32_t n_atoms, const float* ali
     if (rc) return rc;
     Launch l;
     if ((rc = plan<Kind::Fit>(n_sel, atom_idx != nullptr, &l))) return rc;
+    if (!align_xyz) {
+        bool done = false;
+        rc = superpose_one_pass(s, xyz, n_frames, n_atoms, atom_idx, n_sel, ref_sel, stats,
+                                (int)(translate != 0), rot_out, rmsd_out, &done);
+        if (rc || done) return rc;
+    }
     const float* fit = align_xyz ? align_xyz : xyz;
     const long long stride = 3LL * n_align_atoms;
     const DeviceInfo* d = current_device();
