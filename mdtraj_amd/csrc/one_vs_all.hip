@@ -105,6 +105,33 @@ __global__ __launch_bounds__(CuGroup<kMinWaves>::kThreads, kMinWaves) void frame
         lane);
 }
 
+// Hands the n words at src (4-byte aligned) to put4(i, four words from i on) and
+// put(i, word i) for the last ones, kLoads loads of 16 bytes a lane in flight.
+// The loads are unconditional (past the end the last unit again): a load
+// under a branch is waited for where the branch ends.
+typedef float V4f __attribute__((ext_vector_type(4), aligned(4)));
+
+template <int kThreads, int kLoads, typename Put4, typename Put>
+__device__ __forceinline__ void copy_words(const float* __restrict__ src, int n, int tid,
+                                           Put4 put4, Put put) {
+    const int whole = n & ~3;
+    float last = 0.0f;
+    if (tid < n - whole) last = src[whole + tid];
+    for (int i0 = 0; i0 < whole; i0 += 4 * kLoads * kThreads) {
+        V4f v[kLoads];
+#pragma unroll
+        for (int t = 0; t < kLoads; ++t)
+            v[t] = __builtin_nontemporal_load(reinterpret_cast<const V4f*>(
+                src + min(i0 + 4 * (t * kThreads + tid), whole - 4)));
+#pragma unroll
+        for (int t = 0; t < kLoads; ++t) {
+            const int i = i0 + 4 * (t * kThreads + tid);
+            if (i < whole) put4(i, v[t]);
+        }
+    }
+    if (tid < n - whole) put(whole + tid, last);
+}
+
 // In-place centering and traces, one wave per frame (two passes over the
 // frame; the second usually hits in L2).  Rounding as the reference:
 // double sums, float mean, float subtraction, float squares summed in double.
@@ -199,13 +226,11 @@ __global__ __launch_bounds__(kBlock) void apply_kernel(float* __restrict__ xyz, 
 //          long (the fit stays in registers), else atoms dealt out flat
 // Rounding is the two kernels': the sums are FP64 in another order.
 //
-// Bound by HBM (a read and a write of every atom) as far as four workgroups of
-// a CU, at different steps, keep it busy: 20,000 frames of 3,001 atoms (375 of
-// them fitted), 1.44 GB, in 366 us (3.9 TB/s) against 390 us for two kernels,
-// which move 2.3 GB.  (Two persistent workgroups a CU, each with a second
-// buffer filled by direct loads to LDS, were slower, 417 us: two frames at
-// work on a CU instead of four.  The sums' indices and reference atoms are
-// asked for ahead of the frames; read where they were used, 398 us.)
+// Bound by HBM, a read and a write of every atom: 20,000 frames of 3,001 atoms
+// (375 of them fitted), 1.44 GB, in 275-325 us by box (4.4-5.2 TB/s, the rate of
+// a device copy) against 390 us for two kernels, which move 2.3 GB.  (Two
+// persistent workgroups a CU, each with a second buffer filled by direct loads
+// to LDS, were slower, 417 us: two frames at work on a CU instead of four.)
 constexpr int kLoads = 10;
 // Frames of this many atoms on keep a frame's fit in registers while whole
 // waves move its atoms.
@@ -223,7 +248,6 @@ __global__ __launch_bounds__(kBlock, 4) void superpose_kernel(
     const int* __restrict__ idx, int n_sel, const float* __restrict__ ref_sel,
     const double* __restrict__ ref_stats, int translate, float* __restrict__ rot_out,
     float* __restrict__ rmsd_out) {
-    typedef float V4f __attribute__((ext_vector_type(4), aligned(4)));
     static_assert(kWavesPer == 1 || kRL == kWave, "waves share frames as whole rows");
     constexpr int kThreads = kBlock;
     constexpr int kNS = SumsPerFrame<Kind::Fit>::value;
@@ -261,25 +285,9 @@ __global__ __launch_bounds__(kBlock, 4) void superpose_kernel(
     };
     fetch(0, a_item);
 
-    for (int i0 = 4 * tid; i0 < n_words; i0 += 4 * kLoads * kThreads) {
-        V4f v[kLoads];
-#pragma unroll
-        for (int t = 0; t < kLoads; ++t) {
-            // past the run's end: its last 16 bytes again (a run has at least
-            // four words unless it is one atom)
-            const int i = min(i0 + 4 * t * kThreads, max(n_words - 4, 0));
-            if (n_words >= 4) v[t] = *reinterpret_cast<const V4f*>(run + i);
-        }
-#pragma unroll
-        for (int t = 0; t < kLoads; ++t) {
-            const int i = i0 + 4 * t * kThreads;
-            if (i + 4 <= n_words) {
-                *reinterpret_cast<float4*>(s_x + i) = make_float4(v[t].x, v[t].y, v[t].z, v[t].w);
-            } else if (i < n_words) {
-                for (int k = i; k < n_words; ++k) s_x[k] = run[k];
-            }
-        }
-    }
+    copy_words<kThreads, kLoads>(run, n_words, tid, [&](int i, V4f v) {
+        *reinterpret_cast<float4*>(s_x + i) = make_float4(v.x, v.y, v.z, v.w);
+    }, [&](int i, float v) { s_x[i] = v; });
     __syncthreads();
 
     // the row's items in turn: frame after frame, item after item; while one is
@@ -546,44 +554,62 @@ int launch_superpose_v(hipStream_t s, float* xyz, long long n_frames, int n_atom
                        const int* idx, int n_sel, const float* ref_sel, const double* stats,
                        int translate, float* rot_out, float* rmsd_out) {
     const long long blocks = (n_frames + per_group - 1) / per_group;
+    const size_t lds = superpose_lds(per_group, kWavesPer, n_atoms);
+    if (lds > 64 * 1024)
+        HR_CHECK_HIP(hipFuncSetAttribute(
+            reinterpret_cast<const void*>(superpose_kernel<kRL, kWavesPer, kGather>),
+            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     hipLaunchKernelGGL((superpose_kernel<kRL, kWavesPer, kGather>), dim3((unsigned)blocks),
-                       dim3(kBlock), superpose_lds(per_group, kWavesPer, n_atoms), s, xyz,
+                       dim3(kBlock), lds, s, xyz,
                        n_frames, n_atoms, per_group, idx, n_sel, ref_sel, stats, translate,
                        rot_out, rmsd_out);
     return launch_status("superpose_kernel");
 }
 
-// One-pass superposition where it is the faster one; *done is false, and
-// nothing is launched, where the two-kernel path is to be used.
+// One-pass superposition where at least two workgroups a CU fit LDS (frames of
+// up to ~6,600 atoms); *done is false, and nothing is launched, where the
+// two-kernel path is to be used.
+//
+// The frames of a run: as many bytes of frames on the way per CU as its LDS and
+// four workgroups allow, whole rounds of rows (or of waves) preferred, the
+// smaller run where that is the same.  Kernel us for 1.44 GB, by run: 8 atoms
+// 64 frames 804, 128 557, 192 533; 22 atoms 64 411, 128 426, 151 456; 50 atoms
+// 32 374, 64 330; 100 atoms 16 412, 32 313; 191 atoms 12 312, 16 293; 420 atoms
+// 4 350, 7 338, 8 319; 606 atoms 4 312, 5 372, 8 369; 850 atoms 3 357, 4 307;
+// 1,700 atoms 1 388, 2 311; 2,000 atoms 1 346, 2 297; 3,001 atoms 1 274, 2 275.
+// (The two kernels: 8 atoms 3,303, 22 atoms 1,470, 100 atoms 575, 300 atoms 497,
+// 606 atoms 455, 1,000 atoms 415, 2,000 atoms 427, 3,001 atoms 390, 4,000 atoms
+// 380, 6,500 atoms 454 us, against 354 in one pass; with a single workgroup a
+// CU, 8,000 atoms, one pass takes 430 us against 387.)
 int superpose_one_pass(hipStream_t s, float* xyz, long long n_frames, int n_atoms, const int* idx,
                        int n_sel, const float* ref_sel, const double* stats, int translate,
                        float* rot_out, float* rmsd_out, bool* done) {
     *done = false;
-    constexpr size_t kLds = 40 * 1000;  // four workgroups a CU
-    auto fits = [&](int group, int waves) { return superpose_lds(group, waves, n_atoms) <= kLds; };
-    int group = 1, waves = 4;
-    if (fits(8, 1)) {
-        group = 8;
-        while (group < kBlock && fits(group + 1, 1)) ++group;
-        waves = 1;
-    } else if (fits(3, 1)) {
-        group = fits(4, 1) ? 4 : 3;
-        waves = 1;
-    } else if (fits(2, 2)) {
-        group = 2;
-        waves = 2;
+    const DeviceInfo* d = current_device();
+    if (!d) return HR_ERR_HIP;
+    const size_t cu = std::min((size_t)160000, d->lds_per_cu);  // in whole pieces
+    int group = 0, waves = 0, rl = 0;
+    double best = 0.0;
+    for (int g = 1; g <= kBlock; g += g < 4 ? 1 : 4) {
+        const int w = g == 1 ? 4 : g == 2 ? 2 : 1;
+        const size_t lds = superpose_lds(g, w, n_atoms);
+        const size_t resident = std::min((size_t)4, cu / lds);
+        if (resident < 2) break;
+        // lanes per frame: by the selection, and no fewer than leave every row
+        // of the workgroup a frame
+        int lanes = n_sel < 28 ? 4 : n_sel < 112 ? 8 : n_sel < 360 ? 16 : kWave;
+        while (lanes < kWave && kBlock / lanes > g) lanes *= 2;
+        const int rows = kBlock / lanes;
+        const double used = w > 1 ? 1.0 : (double)g / ((g + rows - 1) / rows * rows);
+        const double score = (double)resident * g * used * used;
+        if (score > best) {
+            best = score;
+            group = g;
+            waves = w;
+            rl = lanes;
+        }
     }
-    // Runs that leave much of their LDS empty keep too few bytes on the way, and
-    // the two kernels are the faster ones (us, one pass against two, 1.44 GB:
-    // 420 atoms, 20 KB runs 511 / 462; 1,000 atoms, 36 KB 396 / 415; 1,700,
-    // 20 KB 512 / 436; 2,000, 24 KB 467 / 413; 2,700, 32 KB 406 / 420; 3,001,
-    // 36 KB 366 / 390); so are they for frames that do not fit at all.  Runs of
-    // many short frames always pay, as apply_kernel takes a workgroup per frame:
-    // 8 atoms 704 / 3,303, 22 atoms 522 / 1,470, 100 atoms 414 / 575, 300 atoms
-    // 409 / 497, 400 atoms 415 / 447.
-    const bool full = group >= 8 || 12LL * group * n_atoms >= 32000;
-    if (!full || !fits(group, waves) || (n_frames + group - 1) / group > INT_MAX) return HR_OK;
-    const int rl = n_sel < 28 ? 4 : n_sel < 112 ? 8 : n_sel < 360 ? 16 : 64;
+    if (!group || (n_frames + group - 1) / group > INT_MAX) return HR_OK;
     *done = true;
 #define HR_SUP(RL, W)                                                                           \
     (idx ? launch_superpose_v<RL, W, true>(s, xyz, n_frames, n_atoms, group, idx, n_sel,        \
@@ -593,6 +619,7 @@ int superpose_one_pass(hipStream_t s, float* xyz, long long n_frames, int n_atom
     if (waves == 4) return HR_SUP(kWave, 4);
     if (waves == 2) return HR_SUP(kWave, 2);
     return rl == 64   ? HR_SUP(64, 1)
+           : rl == 32 ? HR_SUP(32, 1)
            : rl == 16 ? HR_SUP(16, 1)
            : rl == 8  ? HR_SUP(8, 1)
                       : HR_SUP(4, 1);
@@ -864,10 +891,10 @@ int hr_rmsd_one_vs_all_prepared(const float* target, int64_t n_frames, int32_t n
     const char* ws = static_cast<const char*>(workspace);
     const double* stats = reinterpret_cast<const double*>(ws);
     const float* ref_sel = reinterpret_cast<const float*>(ws + kRefOffset);
+    hipStream_t s = (hipStream_t)stream;
     Launch l;
     int rc = plan<Kind::Rmsd>(n_sel, atom_idx != nullptr, &l);
     if (rc) return rc;
-    hipStream_t s = (hipStream_t)stream;
     const long long stride = 3LL * n_atoms_total;
     if (atom_idx)
         return launch_frames<Kind::Rmsd, false, true>(l, s, target, n_frames, stride, 0, atom_idx,

@@ -15,7 +15,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("n_atoms", [1, 2, 3, 21, 22, 27, 28, 112, 191, 192, 400, 416, 420, 700,
                                      830, 1000, 1111, 1400, 1650, 1700, 2000, 2700, 3001, 3320,
-                                     3400])
+                                     3400, 4450, 6600, 6700])
 @pytest.mark.parametrize("n_frames", [1, 7, 301])
 def test_sizes(gpu, n_atoms, n_frames):
     if n_atoms * n_frames > 300000:
