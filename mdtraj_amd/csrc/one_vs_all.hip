@@ -132,6 +132,67 @@ __device__ __forceinline__ void copy_words(const float* __restrict__ src, int n,
     if (tid < n - whole) put(whole + tid, last);
 }
 
+// One-vs-all over whole short frames: a lane per frame.  A wave's 64 frames
+// are consecutive in memory; they come into LDS 16 bytes a lane, and each
+// lane then walks its own frame there, the reference atoms being the same for
+// all lanes (scalar loads).  There is nothing to reduce across lanes and no
+// lane without an atom, which is what bounds rows of 4 or 8 lanes on such
+// frames (vector instructions per 22-atom frame: about 37 a wave, here 17).
+// Bank conflicts: lane strides of 3 n words, n a multiple of 4, would meet in
+// 16 banks or fewer, so such frames are spread by a word each.
+//
+// Us per launch with the reference's preparation, rows of lanes against a lane
+// per frame: 2,000,003 frames of 8 atoms 97 / 61; 1,000,003 of 12 57 / 34, of 16
+// 61 / 43, of 22 92 / 64, of 30 98 / 87; 700,000 of 36 102 / 77; 500,000 of 40 80 /
+// 67, of 45 80 / 81, of 52 83 / 91; 1,000 frames of 22 13 / 10, of 8 11 / 7.  With
+// 64 frames in LDS a wave, longer frames leave the CU too few waves; hence
+// kShortAtoms.  At 22 atoms HBM would allow 41 us (264 MB); the rest is the
+// sums' and the fits' FP64 work, about 28 us of vector issue, and the nine
+// waves a CU's LDS holds.
+constexpr int kShortLoads = 9;
+constexpr int kShortAtoms = 40;
+
+__global__ __launch_bounds__(kWave, 3) void short_frames_kernel(
+    const float* __restrict__ xyz, long long n_frames, int n_atoms,
+    const float* __restrict__ ref_sel, const double* __restrict__ ref_stats, long long self_frame,
+    float* __restrict__ out) {
+    extern __shared__ __align__(16) float s_frames[];
+    const int lane = threadIdx.x;
+    const long long f0 = (long long)blockIdx.x * kWave;
+    const int cnt = (int)min((long long)kWave, n_frames - f0);
+    const int words = 3 * n_atoms, n_words = cnt * words;
+    const bool spread = (n_atoms & 3) == 0;
+    const float* run = xyz + f0 * words;
+    // frame of 16-byte unit u when frames are whole units: u / (words / 4)
+    const unsigned magic = 0xFFFFFFFFu / (unsigned)max(words / 4, 2) + 1u;
+    copy_words<kWave, kShortLoads>(run, n_words, lane, [&](int i, V4f v) {
+        if (spread) {
+            float* to = s_frames + i + (int)__umulhi((unsigned)i / 4, magic);
+            to[0] = v.x;
+            to[1] = v.y;
+            to[2] = v.z;
+            to[3] = v.w;
+        } else {
+            *reinterpret_cast<float4*>(s_frames + i) = make_float4(v.x, v.y, v.z, v.w);
+        }
+    }, [&](int i, float v) { s_frames[i] = v; });  // (frames of whole units end on one)
+    __syncthreads();
+    if (lane >= cnt) return;
+    const float* fr = s_frames + lane * (words + (spread ? 1 : 0));
+    Sums s = {};
+#pragma unroll 4
+    for (int j = 0; j < n_atoms; ++j)
+        accumulate<Kind::Rmsd>(s, fr[3 * j], fr[3 * j + 1], fr[3 * j + 2], ref_sel[j],
+                               ref_sel[n_atoms + j], ref_sel[2 * n_atoms + j]);
+    const double rs[4] = {ref_stats[0], ref_stats[1], ref_stats[2], ref_stats[3]};
+    const double n = (double)n_atoms;
+    double M[9], ga, gb;
+    centred(s, rs, n, M, ga, gb);
+    const double msd = qcp_msd(M, ga, gb, n);
+    const long long f = f0 + lane;
+    out[f] = f == self_frame ? 0.0f : (float)sqrt(msd);
+}
+
 // In-place centering and traces, one wave per frame (two passes over the
 // frame; the second usually hits in L2).  Rounding as the reference:
 // double sums, float mean, float subtraction, float squares summed in double.
@@ -892,6 +953,13 @@ int hr_rmsd_one_vs_all_prepared(const float* target, int64_t n_frames, int32_t n
     const double* stats = reinterpret_cast<const double*>(ws);
     const float* ref_sel = reinterpret_cast<const float*>(ws + kRefOffset);
     hipStream_t s = (hipStream_t)stream;
+    if (!atom_idx && n_sel <= kShortAtoms && n_frames <= (long long)INT_MAX * kWave) {
+        const size_t lds = (size_t)kWave * (12 * n_sel + 4);
+        hipLaunchKernelGGL(short_frames_kernel, dim3((unsigned)((n_frames + kWave - 1) / kWave)),
+                           dim3(kWave), lds, s, target, (long long)n_frames, n_sel, ref_sel, stats,
+                           (long long)self_frame, out);
+        return launch_status("short_frames_kernel");
+    }
     Launch l;
     int rc = plan<Kind::Rmsd>(n_sel, atom_idx != nullptr, &l);
     if (rc) return rc;
