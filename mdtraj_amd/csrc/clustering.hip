@@ -9,7 +9,8 @@
 //            16-byte loads in flight per lane); one workgroup adds them in order and
 //            forms the population std of the n^2 entries: mean = 2 S1 / n^2,
 //            var = 2 S2 / n^2 - mean^2.
-//   tiles    one pass over 256 x 256 tiles of the upper triangle: the lane of
+//   tiles    one pass over tiles of 256 columns by 32 or 64 rows of the upper
+//            triangle: the lane of
 //            column j walks the tile's rows i (each row's 256 entries are
 //            consecutive in the condensed layout), so every entry's affinity
 //            is computed once and added to its column in the lane's register
@@ -26,7 +27,7 @@ namespace {
 constexpr int kCBlock = 256;
 constexpr int kStatBlocks = 4096;
 constexpr int kStatUnroll = 8;
-constexpr int kCTile = 256;    // rows and columns of a score tile (one lane per column)
+constexpr int kCTile = 256;    // columns of a score tile, one lane each
 constexpr int kRowBatch = 8;   // rows whose loads are issued together (rows8_sum)
 
 __host__ __device__ __forceinline__ long long cidx(long long i, long long j, long long n) {
@@ -139,19 +140,29 @@ __device__ __forceinline__ double rows8_sum(const double (&a)[8], int lane) {
     return e;
 }
 
-// Tile (bi, bj), bj >= bi, of the score matrix: rows bi*kCTile.., columns
-// bj*kCTile..; row_part[bj * n + i] and col_part[bi * n + j].
+// Rows of a tile, which has 256 columns: few enough that the tiles fill the
+// chip.  Us of hr_centroid_scores with tiles of 256 rows, as many as columns,
+// and with these: 1,000 frames 78 / 27, 4,001 84 / 59, 8,000 174 / 154, 12,000
+// 274 / 202, 16,100 464 / 346.  32 and 64 rows are even at 8,000 frames; beyond,
+// the fewer column partials are the better.
+constexpr int kTallTile = 64, kLowTile = 32;
+constexpr long long kLowTileFrames = 8064;
+
+// Tile (bi, bj) of the score matrix: rows bi*kTileRows.., columns bj*kCTile..,
+// unless it is all on or below the diagonal; row_part[bj * n + i] and
+// col_part[bi * n + j].
+template <int kTileRows>
 __global__ __launch_bounds__(kCBlock) void centroid_tile_kernel(
     const float* __restrict__ d, long long n, double neg_beta, const double* __restrict__ stats,
     double* __restrict__ row_part, double* __restrict__ col_part) {
     const int bi = blockIdx.y, bj = blockIdx.x;
-    if (bj < bi) return;  // whole workgroup: the lower triangle of tiles
-    __shared__ double rows[kCBlock / kWave][kCTile];
+    if (bj < (long long)bi * kTileRows / kCTile) return;  // whole workgroup
+    __shared__ double rows[kCBlock / kWave][kTileRows];
     const double k_aff = neg_beta / stats[2];
     const int w = threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1);
-    const long long i0 = (long long)bi * kCTile;
+    const long long i0 = (long long)bi * kTileRows;
     const long long j = (long long)bj * kCTile + threadIdx.x;
-    const int n_rows = (int)(n - i0 < kCTile ? n - i0 : kCTile);
+    const int n_rows = (int)(n - i0 < kTileRows ? n - i0 : kTileRows);
     double col = 0.0;
     if (n < 2) {  // no entries (and maybe no matrix): one tile of zero partials
         if (threadIdx.x < n_rows) row_part[(long long)bj * n + i0 + threadIdx.x] = 0.0;
@@ -191,21 +202,38 @@ __global__ __launch_bounds__(kCBlock) void centroid_tile_kernel(
     if (j < n) col_part[(long long)bi * n + j] = col;
 }
 
-__global__ __launch_bounds__(kCBlock) void centroid_finish_kernel(
+// Frame i's score: its row's partial of every column tile from its own on, and
+// its column's partial of every row tile that reaches above the diagonal there,
+// eight loads in flight.
+__global__ __launch_bounds__(kWave) void centroid_finish_kernel(
     const double* __restrict__ row_part, const double* __restrict__ col_part, long long n,
-    int n_tiles, double* __restrict__ scores) {
-    const long long i = (long long)blockIdx.x * kCBlock + threadIdx.x;
+    int n_tiles, int tile_rows, double* __restrict__ scores) {
+    const long long i = (long long)blockIdx.x * kWave + threadIdx.x;
     if (i >= n) return;
+    constexpr int kEach = 8;
+    auto add = [&](double s, const double* part, int t0, int t1) {
+        for (int t = t0; t < t1; t += kEach) {
+            double v[kEach];
+#pragma unroll
+            for (int u = 0; u < kEach; ++u) v[u] = part[(long long)min(t + u, t1 - 1) * n + i];
+#pragma unroll
+            for (int u = 0; u < kEach; ++u)
+                if (t + u < t1) s += v[u];
+        }
+        return s;
+    };
     const int b = (int)(i / kCTile);
+    const int n_rows = (int)((n + tile_rows - 1) / tile_rows);
     double s = 1.0;  // the diagonal: exp(0)
-    for (int t = b; t < n_tiles; ++t) s += row_part[(long long)t * n + i];
-    for (int t = 0; t <= b; ++t) s += col_part[(long long)t * n + i];
+    s = add(s, row_part, b, n_tiles);
+    s = add(s, col_part, 0, min(n_rows, ((b + 1) * kCTile - 2) / tile_rows + 1));
     scores[i] = s;
 }
 
 size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 
 int score_tiles(long long n) { return (int)((n + kCTile - 1) / kCTile); }
+int score_tile_rows(long long n) { return n < kLowTileFrames ? kLowTile : kTallTile; }
 
 }  // namespace
 }  // namespace hr
@@ -217,7 +245,9 @@ extern "C" {
 size_t hr_centroid_workspace_bytes(int64_t n_frames) {
     const long long n = n_frames > 0 ? n_frames : 1;
     return align256(2 * kStatBlocks * sizeof(double)) + align256(4 * sizeof(double)) +
-           2 * align256((size_t)score_tiles(n) * n * sizeof(double));
+           align256((size_t)score_tiles(n) * n * sizeof(double)) +
+           align256((size_t)((n + score_tile_rows(n) - 1) / score_tile_rows(n)) * n *
+                    sizeof(double));
 }
 
 int hr_centroid_scores(const float* condensed, int64_t n_frames, double beta, double* scores,
@@ -228,7 +258,7 @@ int hr_centroid_scores(const float* condensed, int64_t n_frames, double beta, do
     HR_REQUIRE(scores && workspace && (condensed || n_frames == 1), "NULL pointer argument");
     HR_REQUIRE((reinterpret_cast<uintptr_t>(condensed) & 15) == 0,
                "condensed must be 16-byte aligned");
-    HR_REQUIRE(score_tiles(n_frames) < 65536, "too many frames (%lld)", (long long)n_frames);
+    HR_REQUIRE(n_frames / score_tile_rows(n_frames) < 65535, "too many frames (%lld)", (long long)n_frames);
     if (!current_device()) return HR_ERR_HIP;
     hipStream_t s = (hipStream_t)stream;
     const long long n = n_frames;
@@ -248,12 +278,14 @@ int hr_centroid_scores(const float* condensed, int64_t n_frames, double beta, do
     if (rc) return rc;
     hipLaunchKernelGGL(centroid_stats_final_kernel, dim3(1), dim3(kCBlock), 0, s, partial, n, st);
     if ((rc = launch_status("centroid_stats_final_kernel"))) return rc;
-    hipLaunchKernelGGL(centroid_tile_kernel, dim3((unsigned)tiles, (unsigned)tiles), dim3(kCBlock),
-                       0, s, condensed, n, -beta, st, row_part, col_part);
+    const int tile_rows = score_tile_rows(n);
+    const auto tile = tile_rows == kTallTile ? centroid_tile_kernel<kTallTile>
+                                             : centroid_tile_kernel<kLowTile>;
+    hipLaunchKernelGGL(tile, dim3((unsigned)tiles, (unsigned)((n + tile_rows - 1) / tile_rows)),
+                       dim3(kCBlock), 0, s, condensed, n, -beta, st, row_part, col_part);
     if ((rc = launch_status("centroid_tile_kernel"))) return rc;
-    const unsigned blocks = (unsigned)((n + kCBlock - 1) / kCBlock);
-    hipLaunchKernelGGL(centroid_finish_kernel, dim3(blocks), dim3(kCBlock), 0, s, row_part,
-                       col_part, n, tiles, scores);
+    hipLaunchKernelGGL(centroid_finish_kernel, dim3((unsigned)((n + kWave - 1) / kWave)),
+                       dim3(kWave), 0, s, row_part, col_part, n, tiles, tile_rows, scores);
     if ((rc = launch_status("centroid_finish_kernel"))) return rc;
     if (stats) {
         HR_CHECK_HIP(hipMemcpyAsync(stats, st, 3 * sizeof(double), hipMemcpyDeviceToDevice, s));
