@@ -40,6 +40,7 @@ class XTCTrajectoryFile:
             raise IOError(f"The file '{self.filename}' doesn't exist")
         self._host = np.fromfile(self.filename, dtype=np.uint8)
         self._dev = None
+        self._dev_offs = None
         load()
         n_frames, n_atoms = ctypes.c_int64(), ctypes.c_int32()
         buf = self._host.ctypes.data_as(ctypes.c_void_p)
@@ -83,6 +84,7 @@ class XTCTrajectoryFile:
 
     def close(self):
         self._dev = None
+        self._dev_offs = None
         self.is_open = False
 
     def __enter__(self):
@@ -119,7 +121,7 @@ class XTCTrajectoryFile:
                 xyz = self._select_atoms(xyz, sel)
         if frames.size:
             self.frame_counter = int(min(len(self), frames[-1] + stride))
-        if np.all(np.logical_and(box < 1e-10, box > -1e-10)):
+        if box.size == 0 or max(box.max(), -box.min()) < 1e-10:
             box = None
         return (xyz if device else dev.to_host(xyz)), time, step, box
 
@@ -141,28 +143,40 @@ class XTCTrajectoryFile:
                  out.data_ptr(), dev.stream())
         return out
 
+    def _device_offsets(self, frames):
+        """Byte offsets of `frames` on the device: part of the file's whole
+        list, kept with its bytes, when they are consecutive."""
+        F = int(frames.size)
+        if int(frames[-1]) - int(frames[0]) != F - 1:
+            return dev.to_device(self._offsets[frames], np.int64)
+        if self._dev_offs is None or dev.is_torch_cuda(self._dev_offs) != dev.is_torch_mode():
+            self._dev_offs = dev.to_device(self._offsets, np.int64)
+        return self._dev_offs[int(frames[0]):int(frames[0]) + F]
+
     def _decode(self, frames):
         F, N = int(frames.size), self.n_atoms
         xyz = dev.empty((F, N, 3), np.float32)
-        time = dev.empty(F, np.float32)
-        step = dev.empty(F, np.int32)
-        box = dev.empty((F, 3, 3), np.float32)
-        prec = dev.empty(F, np.float32)
-        status = dev.empty(F, np.int32)
+        # time, step, box, precision and status share a buffer: one copy to the
+        # host where five would each wait for the device (with the kept offsets
+        # 459 -> 377 us a read of 10,000 frames x 3,001 atoms)
+        meta = dev.empty(13 * F, np.float32)
         if F:
             data = self._device_bytes()
-            offs = dev.to_device(self._offsets[frames], np.int64)
+            offs = self._device_offsets(frames)
+            part = [meta.data_ptr() + 4 * F * k for k in (0, 1, 2, 11, 12)]
             call("hr_xtc_decode", data.data_ptr(), data.numel(), offs.data_ptr(), F, N,
-                 xyz.data_ptr(), time.data_ptr(), step.data_ptr(), box.data_ptr(),
-                 prec.data_ptr(), status.data_ptr(), dev.stream())
-            st = dev.to_host(status)
-            bad = np.flatnonzero(st)
-            if bad.size:
-                f = int(frames[bad[0]])
-                raise RuntimeError(f"XTC read error: {_STATUS.get(int(st[bad[0]]), 'unknown')} "
-                                   f"(frame {f})")
-        self.last_precision = dev.to_host(prec)
-        return xyz, dev.to_host(time), dev.to_host(step), dev.to_host(box)
+                 xyz.data_ptr(), *part, dev.stream())
+        host = dev.to_host(meta)
+        time, step, box, prec, st = (host[F * i:F * k] for i, k in
+                                     ((0, 1), (1, 2), (2, 11), (11, 12), (12, 13)))
+        bad = np.flatnonzero(st.view(np.int32))
+        if bad.size:
+            f = int(frames[bad[0]])
+            raise RuntimeError("XTC read error: "
+                               f"{_STATUS.get(int(st.view(np.int32)[bad[0]]), 'unknown')} "
+                               f"(frame {f})")
+        self.last_precision = prec
+        return xyz, time, step.view(np.int32), box.reshape(F, 3, 3)
 
 
 def load_xtc(filename, top=None, stride=None, atom_indices=None, frame=None):
