@@ -152,6 +152,11 @@ __device__ __forceinline__ void copy_words(const float* __restrict__ src, int n,
 constexpr int kShortLoads = 9;
 constexpr int kShortAtoms = 40;
 
+// kRawRef: ref_sel is the reference itself (x, y, z interleaved) and every wave
+// prepares it, with ref_prep_body's arithmetic (each of its first n_atoms
+// threads has one atom), into LDS: the one launch of a small host call, where
+// frames and reference are read over PCIe.
+template <bool kRawRef>
 __global__ __launch_bounds__(kWave, 3) void short_frames_kernel(
     const float* __restrict__ xyz, long long n_frames, int n_atoms,
     const float* __restrict__ ref_sel, const double* __restrict__ ref_stats, long long self_frame,
@@ -163,6 +168,13 @@ __global__ __launch_bounds__(kWave, 3) void short_frames_kernel(
     const int words = 3 * n_atoms, n_words = cnt * words;
     const bool spread = (n_atoms & 3) == 0;
     const float* run = xyz + f0 * words;
+    __shared__ float s_ref[kRawRef ? 3 * kShortAtoms : 1];
+    float ref_x = 0.0f, ref_y = 0.0f, ref_z = 0.0f;
+    if (kRawRef && lane < n_atoms) {
+        ref_x = ref_sel[3 * lane];
+        ref_y = ref_sel[3 * lane + 1];
+        ref_z = ref_sel[3 * lane + 2];
+    }
     // frame of 16-byte unit u when frames are whole units: u / (words / 4)
     const unsigned magic = 0xFFFFFFFFu / (unsigned)max(words / 4, 2) + 1u;
     copy_words<kWave, kShortLoads>(run, n_words, lane, [&](int i, V4f v) {
@@ -176,15 +188,33 @@ __global__ __launch_bounds__(kWave, 3) void short_frames_kernel(
             *reinterpret_cast<float4*>(s_frames + i) = make_float4(v.x, v.y, v.z, v.w);
         }
     }, [&](int i, float v) { s_frames[i] = v; });  // (frames of whole units end on one)
+    double rs[4];
+    const float* rx = ref_sel;
+    if constexpr (kRawRef) {
+        if (lane < n_atoms) {
+            s_ref[lane] = ref_x;
+            s_ref[n_atoms + lane] = ref_y;
+            s_ref[2 * n_atoms + lane] = ref_z;
+        }
+        const double x = ref_x, y = ref_y, z = ref_z;
+        rs[0] = wave_sum(x);
+        rs[1] = wave_sum(y);
+        rs[2] = wave_sum(z);
+        rs[3] = wave_sum(fma(x, x, fma(y, y, fma(z, z, 0.0))));
+        rx = s_ref;
+    } else {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) rs[c] = ref_stats[c];
+    }
     __syncthreads();
     if (lane >= cnt) return;
     const float* fr = s_frames + lane * (words + (spread ? 1 : 0));
+    const float* ry = rx + n_atoms;
+    const float* rz = ry + n_atoms;
     Sums s = {};
 #pragma unroll 4
     for (int j = 0; j < n_atoms; ++j)
-        accumulate<Kind::Rmsd>(s, fr[3 * j], fr[3 * j + 1], fr[3 * j + 2], ref_sel[j],
-                               ref_sel[n_atoms + j], ref_sel[2 * n_atoms + j]);
-    const double rs[4] = {ref_stats[0], ref_stats[1], ref_stats[2], ref_stats[3]};
+        accumulate<Kind::Rmsd>(s, fr[3 * j], fr[3 * j + 1], fr[3 * j + 2], rx[j], ry[j], rz[j]);
     const double n = (double)n_atoms;
     double M[9], ga, gb;
     centred(s, rs, n, M, ga, gb);
@@ -463,6 +493,15 @@ __global__ __launch_bounds__(kBlock, 4) void superpose_kernel(
     }
 }
 
+template <bool kRawRef>
+int launch_short(hipStream_t s, const float* xyz, long long n_frames, int n_atoms,
+                 const float* ref, const double* stats, long long self_frame, float* out) {
+    hipLaunchKernelGGL(short_frames_kernel<kRawRef>, dim3((unsigned)((n_frames + kWave - 1) / kWave)),
+                       dim3(kWave), (size_t)kWave * (12 * n_atoms + 4), s, xyz, n_frames, n_atoms,
+                       ref, stats, self_frame, out);
+    return launch_status("short_frames_kernel");
+}
+
 struct Launch {
     size_t lds;
     int stage;  // kStageAll, kStageIdx or kStageNone
@@ -594,6 +633,10 @@ int launch_frames(const Launch& l, hipStream_t s, const float* xyz, long long n_
 int one_vs_all_fused_ref(hipStream_t s, const float* frames, long long n_frames, int n_sel,
                          const float* ref, long long self_frame, float* out, bool* done) {
     *done = false;
+    if (n_sel <= kShortAtoms) {
+        *done = true;
+        return launch_short<true>(s, frames, n_frames, n_sel, ref, nullptr, self_frame, out);
+    }
     Launch l;
     int rc = plan<Kind::Rmsd>(n_sel, false, &l);
     if (rc || l.stage != kStageAll) return rc;
@@ -954,11 +997,7 @@ int hr_rmsd_one_vs_all_prepared(const float* target, int64_t n_frames, int32_t n
     const float* ref_sel = reinterpret_cast<const float*>(ws + kRefOffset);
     hipStream_t s = (hipStream_t)stream;
     if (!atom_idx && n_sel <= kShortAtoms && n_frames <= (long long)INT_MAX * kWave) {
-        const size_t lds = (size_t)kWave * (12 * n_sel + 4);
-        hipLaunchKernelGGL(short_frames_kernel, dim3((unsigned)((n_frames + kWave - 1) / kWave)),
-                           dim3(kWave), lds, s, target, (long long)n_frames, n_sel, ref_sel, stats,
-                           (long long)self_frame, out);
-        return launch_status("short_frames_kernel");
+        return launch_short<false>(s, target, n_frames, n_sel, ref_sel, stats, self_frame, out);
     }
     Launch l;
     int rc = plan<Kind::Rmsd>(n_sel, atom_idx != nullptr, &l);
