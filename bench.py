@@ -1004,7 +1004,7 @@ def bench_lprmsd(args):
     """LP-RMSD (md.lprmsd) of a solvated system: 100 distinguishable solute
     atoms and 300 water oxygens whose labels may permute, 20,000 frames of
     400 atoms (the oxygens drift and swap places between frames).  Timed:
-    hr_lprmsd (one wave per frame: fit on the solute, exact assignment of the
+    hr_lprmsd (two waves per frame: fit on the solute, exact assignment of the
     oxygens, QCP), inputs in HBM."""
     import numpy as np
     import torch

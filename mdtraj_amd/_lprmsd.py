@@ -3,7 +3,7 @@
 The RMSD of every target frame to ``reference[frame]``, minimised over the
 rotation and over relabellings of the atoms inside each permute group.  The
 steps, the argument validation and the error messages are the reference's
-(_lprmsd.pyx:232-271).  Per frame, ``hr_lprmsd`` runs one wave:
+(_lprmsd.pyx:232-271).  Per frame, ``hr_lprmsd`` runs two waves:
   (1) centre the selection;
   (2) fit the atoms in no group and rotate by that fit;
   (3) solve each group's assignment exactly (Hungarian method);
