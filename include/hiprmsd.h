@@ -333,7 +333,8 @@ int hr_rmsd_cross(const void* block_a, int64_t n_a, const void* block_b, int64_t
  * std over all n^2 entries
  * (numpy's population std); FP64 throughout; the centroid is the argmax.
  * stats (optional, 3 doubles) receives sum(d_ij, i<j), sum(d_ij^2, i<j) and
- * the std.  Workspace: hr_centroid_workspace_bytes(n).
+ * the std.  Workspace: hr_centroid_workspace_bytes(n), which never falls as n
+ * grows: one sized for the most frames serves fewer.
  * ------------------------------------------------------------------------- */
 size_t hr_rmsd_cross_argmin_workspace_bytes(int64_t n_a);
 int hr_rmsd_cross_argmin(const void* block_a, int64_t n_a, const void* block_b, int64_t n_b,

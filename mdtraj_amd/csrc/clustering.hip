@@ -19,6 +19,8 @@
 //   finish   scores[i] = 1 + the row partials of the tiles right of i's row
 //            block + the column partials of the tiles above i's column block,
 //            in tile order.
+#include <algorithm>
+
 #include "common.h"
 
 namespace hr {
@@ -235,6 +237,15 @@ size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 int score_tiles(long long n) { return (int)((n + kCTile - 1) / kCTile); }
 int score_tile_rows(long long n) { return n < kLowTileFrames ? kLowTile : kTallTile; }
 
+// Bytes hr_centroid_scores uses for n frames: the statistics, then the row
+// tiles' and the column tiles' partial scores.
+size_t workspace_for(long long n) {
+    return align256(2 * kStatBlocks * sizeof(double)) + align256(4 * sizeof(double)) +
+           align256((size_t)score_tiles(n) * n * sizeof(double)) +
+           align256((size_t)((n + score_tile_rows(n) - 1) / score_tile_rows(n)) * n *
+                    sizeof(double));
+}
+
 }  // namespace
 }  // namespace hr
 
@@ -244,10 +255,10 @@ extern "C" {
 
 size_t hr_centroid_workspace_bytes(int64_t n_frames) {
     const long long n = n_frames > 0 ? n_frames : 1;
-    return align256(2 * kStatBlocks * sizeof(double)) + align256(4 * sizeof(double)) +
-           align256((size_t)score_tiles(n) * n * sizeof(double)) +
-           align256((size_t)((n + score_tile_rows(n) - 1) / score_tile_rows(n)) * n *
-                    sizeof(double));
+    // taller tiles from kLowTileFrames on need less than lower ones just below
+    // it, but a workspace for n frames serves fewer than n too
+    return n < kLowTileFrames ? workspace_for(n)
+                              : std::max(workspace_for(n), workspace_for(kLowTileFrames - 1));
 }
 
 int hr_centroid_scores(const float* condensed, int64_t n_frames, double beta, double* scores,
