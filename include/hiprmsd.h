@@ -263,7 +263,8 @@ int hr_rmsd_align_displace(const float* align, int64_t n_frames, int32_t align_s
  *               about the origin when fitted), as md.rmsf does when it is
  *               given atom_indices
  *   out         float32[n_sel]: sqrt(mean_f |x_f - <x>|^2), FP64 sums
- *   workspace   hr_rmsf_workspace_bytes(n_frames, n_sel) bytes
+ *   workspace   hr_rmsf_workspace_bytes(n_frames, n_sel) bytes (never falls as
+ *               either grows: one sized for the largest serves the others)
  * ------------------------------------------------------------------------- */
 size_t hr_rmsf_workspace_bytes(int64_t n_frames, int32_t n_sel);
 int hr_rmsf(const float* xyz, int64_t n_frames, int32_t n_atoms, const int32_t* atom_idx,

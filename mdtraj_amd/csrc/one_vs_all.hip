@@ -926,12 +926,24 @@ __global__ __launch_bounds__(kFinishWaves * kWave) void rmsf_finish_kernel(
 // Frame chunks of the RMSF accumulation: about 2,048 workgroups in all (eight
 // a CU, as many as are resident), at most 1,024 chunks and never more chunks
 // than frames (sizes the workspace, so it depends on the problem only).
+constexpr int kRmsfGroups = 2048, kRmsfMaxChunks = 1024;
+
 int rmsf_chunks(long long n_frames, int n_sel) {
     const long long atom_blocks = (n_sel + kBlock - 1) / kBlock;
-    long long c = (2048 + atom_blocks - 1) / atom_blocks;
-    if (c > 1024) c = 1024;
+    long long c = (kRmsfGroups + atom_blocks - 1) / atom_blocks;
+    if (c > kRmsfMaxChunks) c = kRmsfMaxChunks;
     if (c > n_frames) c = n_frames;
     return (int)(c < 1 ? 1 : c);
+}
+
+// Partial sums (of four doubles) to reserve for rmsf_chunks(n_frames, n_sel) *
+// n_sel.  That product falls where another block of atoms takes chunks away
+// (1,024 x 512 atoms, 683 x 513); with b blocks it is below n_sel (kRmsfGroups /
+// b + 1) <= kRmsfGroups kBlock + n_sel, and this bound grows with both sizes, so
+// that a workspace for many atoms serves fewer.
+size_t rmsf_partials(long long n_frames, int n_sel) {
+    const size_t chunks = (size_t)std::min(n_frames, (long long)kRmsfMaxChunks);
+    return std::min(chunks * n_sel, (size_t)kRmsfGroups * kBlock + n_sel);
 }
 
 // Default chunk of hr_superpose (MiB of coordinates); HR_TUNE_SUPERPOSE_CHUNK_MIB
@@ -1201,8 +1213,7 @@ int hr_rmsd_align_displace(const float* align, int64_t n_frames, int32_t align_s
 size_t hr_rmsf_workspace_bytes(int64_t n_frames, int32_t n_sel) {
     size_t b = hr_superpose_workspace_bytes(n_frames, n_sel);
     b = (b + 255) & ~(size_t)255;
-    b += (size_t)rmsf_chunks(n_frames > 0 ? n_frames : 1, n_sel > 0 ? n_sel : 1) *
-         (size_t)(n_sel > 0 ? n_sel : 0) * 4 * sizeof(double);
+    b += rmsf_partials(n_frames > 0 ? n_frames : 1, n_sel > 0 ? n_sel : 0) * 4 * sizeof(double);
     return b;
 }
 
