@@ -201,6 +201,10 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 // |b|^2 a value (below 3 m) is off by 3 m 2^-19 for its last four bits, by
 // 1.2 m 2^-20 for the product's roundings, and the double cost, of float
 // squares, by m 2^-20: two values by 16.4 m 2^-20 together; tol is twice that.
+// That holds while nothing overflows or goes below float's normal numbers, and
+// the places that fill up the last tile (1e30, less 2 m at most) are farther
+// than any target while 3 m is below 1e30 - 2 m: rows with m outside 2^-96 ..
+// 2^96 (8e28) are all scanned in double.
 // Returns whether every row of the lane has a finite least cost.
 //   q   the group's target atoms as x, z, y, |b|^2, 16-byte aligned
 //   biggest   the largest |b|^2
@@ -269,10 +273,11 @@ __device__ __forceinline__ bool lp_row_minima(const float* q, int k, const float
         const bool mine = half == 0 && r0 + in < k;
         const float* near = q + 4 * min(args[0], k - 1);
         double least = lp_cost(x - near[0], y - near[2], z - near[1]);
-        const float tol = 0x1p-15f * fmaxf(aa, biggest);
+        const float m = fmaxf(aa, biggest), tol = 0x1p-15f * m;
+        const bool plain = m > 0x1p-96f && m < 0x1p96f;
         // the close rows, one by one, the columns spread over the lanes
-        for (unsigned long long close = __ballot(mine && !(second[0] > best[0] + tol)); close;
-             close &= close - 1) {
+        for (unsigned long long close = __ballot(mine && !(plain && second[0] > best[0] + tol));
+             close; close &= close - 1) {
             const int l = __ffsll((long long)close) - 1;
             const float rx = __shfl(x, l, kWave), ry = __shfl(y, l, kWave), rz = __shfl(z, l, kWave);
             double c_best = __builtin_huge_val();

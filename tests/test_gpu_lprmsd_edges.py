@@ -1,0 +1,27 @@
+"""LP-RMSD at the edges of its group search, against the FP64 oracle."""
+import numpy as np
+import pytest
+
+import mdtraj_amd as md
+from oracle import lprmsd as olp
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("scale", [1e16, 1e-17])
+@pytest.mark.parametrize("k,noise", [(33, 0.02), (63, 0.02), (63, 0.6), (70, 0.02)])
+def test_coordinates_of_any_size(gpu, k, noise, scale):
+    """Squared distances beyond the value that fills up the search's last tile
+    of targets (63 atoms leave one such place, 33 leave 31), and below what its
+    float products resolve.  The bar is the 2e-5 of coordinates of order 1."""
+    rng = np.random.default_rng(k)
+    base = np.concatenate([rng.normal(0, 0.6, (7, 3)), rng.uniform(-1, 1, (k, 3))])
+    x = base[None] + rng.normal(0, noise, (3, k + 7, 3))
+    for f in range(3):
+        x[f, 7:] = x[f, 7 + rng.permutation(k)]
+    x = (scale * x).astype(np.float32)
+    ref = (scale * base[None]).astype(np.float32)
+    groups = [np.arange(7, 7 + k)]
+    want = olp.lprmsd(x, ref, 0, None, groups)
+    got = md.lprmsd(x, ref, 0, None, groups)
+    assert np.abs(got - want).max() < 2e-5 * scale
