@@ -48,9 +48,9 @@ __host__ __device__ inline size_t lp_lds_bytes(int n_sel, int kmax) {
            + k1;           // used
 }
 
-// The workgroup is one wave, whose LDS accesses complete in program order:
-// ordering them needs only a wavefront fence that keeps the compiler from
-// moving them, not a workgroup barrier (which would also wait for memory).
+// What only the lead wave touches: a wave's LDS accesses complete in program
+// order, so ordering them needs only a wavefront fence that keeps the compiler
+// from moving them, not a workgroup barrier (which would also wait for memory).
 __device__ __forceinline__ void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
@@ -431,6 +431,7 @@ __global__ __launch_bounds__(kLpFrameBlock, 4) void lp_frame_kernel(LpArgs A) {
 #pragma unroll
             for (int e = 0; e < 9; ++e) s_rot[e] = R1[e];
         }
+        wave_sync();  // read by every lane below, with no group in between where all are empty
     }
 
     // (3) the assignment inside each group

@@ -25,3 +25,22 @@ def test_coordinates_of_any_size(gpu, k, noise, scale):
     want = olp.lprmsd(x, ref, 0, None, groups)
     got = md.lprmsd(x, ref, 0, None, groups)
     assert np.abs(got - want).max() < 2e-5 * scale
+
+
+@pytest.mark.parametrize("groups", [[[]], [[], []]])
+def test_groups_without_atoms(gpu, groups):
+    """No group between the fit on the solute and the final RMSD and rotation,
+    which read it from LDS: the plain RMSD, every frame turned by its own fit."""
+    rng = np.random.default_rng(5)
+    base = rng.normal(0, 0.6, (41, 3))
+    x = base[None] + rng.normal(0, 0.05, (67, 41, 3))
+    for f in range(67):
+        q, _ = np.linalg.qr(rng.normal(size=(3, 3)))
+        x[f] = x[f] @ (q if np.linalg.det(q) > 0 else -q)
+    x = x.astype(np.float32)
+    ref = base[None].astype(np.float32)
+    want, moved = olp.lprmsd(x, ref, 0, None, groups, superpose=True)
+    y = x.copy()
+    got = md.lprmsd(y, ref, 0, permute_groups=groups, superpose=True)
+    assert np.abs(got - want).max() < 2e-5
+    assert np.abs(y - moved).max() < 2e-5
