@@ -61,8 +61,22 @@ inline int launch_status(const char* what) {
     return HR_OK;
 }
 
+// Grid of a kernel that has one workgroup per `groups`, as rows of equal length
+// short enough for a launch: from 2^32 work-items in one dimension on (33.5 M
+// workgroups of 128) the count wraps, and what is past it is left out without an
+// error.  workgroup_index() numbers the workgroups; the last may lie past `groups`.
+inline dim3 launch_grid(long long groups, int threads) {
+    const long long most = 0xFFFFFFFFLL / threads;
+    const long long rows = (groups + most - 1) / most;
+    return dim3((unsigned)((groups + rows - 1) / rows), (unsigned)rows);
+}
+
 // --------------------------------------------------------------- device side
 constexpr int kWave = 64;
+
+__device__ __forceinline__ long long workgroup_index() {
+    return (long long)blockIdx.y * gridDim.x + blockIdx.x;
+}
 
 // Coordinates, references and indices always live in global memory, but a
 // pointer the kernel reads from a descriptor table is generic to the

@@ -328,7 +328,8 @@ __global__ __launch_bounds__(kLpFrameBlock, 4) void lp_frame_kernel(LpArgs A) {
     __shared__ float s_biggest;
     __shared__ float s_rot[9];  // R1
     __shared__ double s_tg;     // the target selection's trace
-    const long long f = blockIdx.x;
+    const long long f = workgroup_index();
+    if (f >= A.n_frames) return;
     float* fr = A.xyz + f * 3LL * A.n_atoms;
     const int n = A.n_sel;
     const float* rx = A.rsel;
@@ -742,7 +743,8 @@ int hr_lprmsd(float* xyz, int64_t n_frames, int32_t n_atoms, const float* ref_fr
         HR_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(lp_frame_kernel),
                                          hipFuncAttributeMaxDynamicSharedMemorySize,
                                          (int)kLpLdsMax));
-    hipLaunchKernelGGL(lp_frame_kernel, dim3((unsigned)n_frames), dim3(kLpFrameBlock), lds, s, A);
+    hipLaunchKernelGGL(lp_frame_kernel, launch_grid(n_frames, kLpFrameBlock), dim3(kLpFrameBlock),
+                       lds, s, A);
     return launch_status("lp_frame_kernel");
 }
 

@@ -44,3 +44,20 @@ def test_groups_without_atoms(gpu, groups):
     got = md.lprmsd(y, ref, 0, permute_groups=groups, superpose=True)
     assert np.abs(got - want).max() < 2e-5
     assert np.abs(y - moved).max() < 2e-5
+
+
+def test_more_frames_than_one_launch_dimension(gpu):
+    """2^25 + 3 frames of two waves each: above 2^32 work-items.  The frames
+    repeat, so every result is one of a few."""
+    free, _ = gpu.cuda.mem_get_info()
+    F, N, some = 2**25 + 3, 3, 7
+    if free < 4 * 12 * F * N:
+        pytest.skip("needs 5 GB of device memory")
+    rng = np.random.default_rng(2)
+    base = rng.uniform(-1, 1, (some, N, 3)).astype(np.float32)
+    x = gpu.from_numpy(base).cuda().repeat(F // some + 1, 1, 1)[:F].contiguous()
+    got = md.lprmsd(x, x[:1], 0, permute_groups=[[1, 2]])
+    few = md.lprmsd(x[:some].clone(), x[:1], 0, permute_groups=[[1, 2]])
+    want = few.repeat(F // some + 1)[:F]
+    assert got.shape == (F,) and bool((got == want).all())
+    assert np.abs(few.cpu().numpy() - olp.lprmsd(base, base[:1], 0, None, [[1, 2]]))[1:].max() < 2e-5
