@@ -163,7 +163,8 @@ __global__ __launch_bounds__(kWave, 3) void short_frames_kernel(
     float* __restrict__ out) {
     extern __shared__ __align__(16) float s_frames[];
     const int lane = threadIdx.x;
-    const long long f0 = (long long)blockIdx.x * kWave;
+    const long long f0 = workgroup_index() * kWave;
+    if (f0 >= n_frames) return;
     const int cnt = (int)min((long long)kWave, n_frames - f0);
     const int words = 3 * n_atoms, n_words = cnt * words;
     const bool spread = (n_atoms & 3) == 0;
@@ -496,9 +497,10 @@ __global__ __launch_bounds__(kBlock, 4) void superpose_kernel(
 template <bool kRawRef>
 int launch_short(hipStream_t s, const float* xyz, long long n_frames, int n_atoms,
                  const float* ref, const double* stats, long long self_frame, float* out) {
-    hipLaunchKernelGGL(short_frames_kernel<kRawRef>, dim3((unsigned)((n_frames + kWave - 1) / kWave)),
-                       dim3(kWave), (size_t)kWave * (12 * n_atoms + 4), s, xyz, n_frames, n_atoms,
-                       ref, stats, self_frame, out);
+    hipLaunchKernelGGL(short_frames_kernel<kRawRef>,
+                       launch_grid((n_frames + kWave - 1) / kWave, kWave), dim3(kWave),
+                       (size_t)kWave * (12 * n_atoms + 4), s, xyz, n_frames, n_atoms, ref, stats,
+                       self_frame, out);
     return launch_status("short_frames_kernel");
 }
 
@@ -1008,9 +1010,8 @@ int hr_rmsd_one_vs_all_prepared(const float* target, int64_t n_frames, int32_t n
     const double* stats = reinterpret_cast<const double*>(ws);
     const float* ref_sel = reinterpret_cast<const float*>(ws + kRefOffset);
     hipStream_t s = (hipStream_t)stream;
-    if (!atom_idx && n_sel <= kShortAtoms && n_frames <= (long long)INT_MAX * kWave) {
+    if (!atom_idx && n_sel <= kShortAtoms)
         return launch_short<false>(s, target, n_frames, n_sel, ref_sel, stats, self_frame, out);
-    }
     Launch l;
     int rc = plan<Kind::Rmsd>(n_sel, atom_idx != nullptr, &l);
     if (rc) return rc;
