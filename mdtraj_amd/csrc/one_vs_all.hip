@@ -7,8 +7,6 @@
 // solve then runs one lane per frame (lane k finishes the k-th frame of the
 // wave's current group of 64).  The reference selection and the atom indices
 // are staged once per workgroup in LDS.
-#include <limits.h>
-
 #include <algorithm>
 
 #include "frames.h"
@@ -351,7 +349,8 @@ __global__ __launch_bounds__(kBlock, 4) void superpose_kernel(
     float* s_x = reinterpret_cast<float*>(s_mem + superpose_head(per_group, kWavesPer));
     const int tid = threadIdx.x, lane = tid & (kWave - 1);
     const int wv = __builtin_amdgcn_readfirstlane(tid / kWave);
-    const long long f0 = (long long)blockIdx.x * per_group;
+    const long long f0 = workgroup_index() * per_group;
+    if (f0 >= n_frames) return;
     const int cnt = (int)min((long long)per_group, n_frames - f0);
     float* run = xyz + f0 * words;
     const int n_words = cnt * words;
@@ -659,16 +658,15 @@ template <int kRL, int kWavesPer, bool kGather>
 int launch_superpose_v(hipStream_t s, float* xyz, long long n_frames, int n_atoms, int per_group,
                        const int* idx, int n_sel, const float* ref_sel, const double* stats,
                        int translate, float* rot_out, float* rmsd_out) {
-    const long long blocks = (n_frames + per_group - 1) / per_group;
+    const long long runs = (n_frames + per_group - 1) / per_group;
     const size_t lds = superpose_lds(per_group, kWavesPer, n_atoms);
     if (lds > 64 * 1024)
         HR_CHECK_HIP(hipFuncSetAttribute(
             reinterpret_cast<const void*>(superpose_kernel<kRL, kWavesPer, kGather>),
             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    hipLaunchKernelGGL((superpose_kernel<kRL, kWavesPer, kGather>), dim3((unsigned)blocks),
-                       dim3(kBlock), lds, s, xyz,
-                       n_frames, n_atoms, per_group, idx, n_sel, ref_sel, stats, translate,
-                       rot_out, rmsd_out);
+    hipLaunchKernelGGL((superpose_kernel<kRL, kWavesPer, kGather>), launch_grid(runs, kBlock),
+                       dim3(kBlock), lds, s, xyz, n_frames, n_atoms, per_group, idx, n_sel,
+                       ref_sel, stats, translate, rot_out, rmsd_out);
     return launch_status("superpose_kernel");
 }
 
@@ -715,7 +713,7 @@ int superpose_one_pass(hipStream_t s, float* xyz, long long n_frames, int n_atom
             rl = lanes;
         }
     }
-    if (!group || (n_frames + group - 1) / group > INT_MAX) return HR_OK;
+    if (!group) return HR_OK;
     *done = true;
 #define HR_SUP(RL, W)                                                                           \
     (idx ? launch_superpose_v<RL, W, true>(s, xyz, n_frames, n_atoms, group, idx, n_sel,        \
