@@ -225,7 +225,7 @@ __global__ __launch_bounds__(kWave, 4) void xtc_decode_kernel(
     __shared__ __align__(16) int s_stage[T::kRows * T::kStage];
     __shared__ int s_magic[kLastIdx];
     const int lane = threadIdx.x, l = lane & (R - 1), row = R == kWave ? 0 : lane / R;
-    const long long f = (long long)blockIdx.x * T::kRows + row;
+    const long long f = workgroup_index() * T::kRows + row;
     for (int i = lane; i < kLastIdx; i += kWave) s_magic[i] = kMagicInts[i];
     xtc_wave_sync();
     uint32_t* ring = s_ring + row * T::kRingRow;
@@ -634,8 +634,8 @@ int hr_xtc_decode(const void* data, int64_t n_bytes, const int64_t* offsets, int
                         : r == 16 ? xtc_decode_kernel<16>
                         : r == 32 ? xtc_decode_kernel<32>
                                   : xtc_decode_kernel<64>;
-    const long long blocks = (n_frames + kWave / r - 1) / (kWave / r);
-    hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(kWave), 0, (hipStream_t)stream,
+    const long long waves = (n_frames + kWave / r - 1) / (kWave / r);
+    hipLaunchKernelGGL(kernel, launch_grid(waves, kWave), dim3(kWave), 0, (hipStream_t)stream,
                        static_cast<const unsigned char*>(data), (long long)n_bytes,
                        reinterpret_cast<const long long*>(offsets), (long long)n_frames, n_atoms,
                        xyz, time, step, box, prec, status);
