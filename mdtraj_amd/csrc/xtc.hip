@@ -211,6 +211,53 @@ inline int xtc_row_lanes(long long n_frames) {
     return n_frames >= 16000 ? 8 : n_frames >= 6000 ? 16 : n_frames >= 3000 ? 32 : 64;
 }
 
+// Frames of up to kTinyAtoms atoms (stored uncompressed, as all of up to nine
+// are): four lanes a frame and nothing in LDS, since the decoder's kernel, with
+// its ring and eight lanes, holds too few of such short frames (us for 1 M frames
+// of 1 / 2 / 3 atoms: 75 / 75 / 86 there, 29 / 34 / 40 here).  Checks and status
+// words as in xtc_decode_kernel.
+constexpr int kTinyAtoms = 3, kTinyLanes = 4, kTinyBlock = 256;
+
+__global__ __launch_bounds__(kTinyBlock) void xtc_tiny_kernel(
+    const unsigned char* __restrict__ data, long long n_bytes,
+    const long long* __restrict__ offsets, long long n_frames, int n_atoms,
+    float* __restrict__ xyz, float* __restrict__ time, int* __restrict__ step,
+    float* __restrict__ box, float* __restrict__ prec, int* __restrict__ status) {
+    const int l = threadIdx.x & (kTinyLanes - 1);
+    const long long f =
+        workgroup_index() * (kTinyBlock / kTinyLanes) + threadIdx.x / kTinyLanes;
+    if (f >= n_frames) return;
+    const long long beg = offsets[f], end = f + 1 < n_frames ? offsets[f + 1] : n_bytes;
+    int st = HR_XTC_OK;
+    if (beg < 0 || end > n_bytes || end - beg < 56 || (beg & 3)) {
+        st = HR_XTC_TRUNCATED;
+    } else {
+        const uint32_t* pw = reinterpret_cast<const uint32_t*>(data + beg);
+        const int magic = (int)be32_word(pw), natoms = (int)be32_word(pw + 1);
+        const int lsize = (int)be32_word(pw + 13);
+        if (l == 0) {
+            step[f] = (int)be32_word(pw + 2);
+            time[f] = __uint_as_float(be32_word(pw + 3));
+        }
+        for (int k = l; k < 9; k += kTinyLanes)
+            box[9 * f + k] = __uint_as_float(be32_word(pw + 4 + k));
+        if (magic != kXtcMagic) {
+            st = HR_XTC_BAD_MAGIC;
+        } else if (natoms != n_atoms || lsize != n_atoms) {
+            st = HR_XTC_ATOMS;
+        } else {
+            if (l == 0) prec[f] = 0.0f;
+            if (14 + 3 * n_atoms > (end - beg) / 4) {
+                st = HR_XTC_TRUNCATED;
+            } else {
+                for (int k = l; k < 3 * n_atoms; k += kTinyLanes)
+                    xyz[3 * n_atoms * f + k] = __uint_as_float(be32_word(pw + 14 + k));
+            }
+        }
+    }
+    if (l == 0) status[f] = st;
+}
+
 // offsets[f] .. offsets[f + 1] (or n_bytes) bound frame f's bytes; the host
 // has checked magic and sizes when it built them.
 template <int R>
@@ -225,7 +272,8 @@ __global__ __launch_bounds__(kWave, 4) void xtc_decode_kernel(
     __shared__ __align__(16) int s_stage[T::kRows * T::kStage];
     __shared__ int s_magic[kLastIdx];
     const int lane = threadIdx.x, l = lane & (R - 1), row = R == kWave ? 0 : lane / R;
-    const long long f = workgroup_index() * T::kRows + row;
+    // wide rows are for few frames (xtc_row_lanes), which one dimension holds
+    const long long f = (R > 8 ? (long long)blockIdx.x : workgroup_index()) * T::kRows + row;
     for (int i = lane; i < kLastIdx; i += kWave) s_magic[i] = kMagicInts[i];
     xtc_wave_sync();
     uint32_t* ring = s_ring + row * T::kRingRow;
@@ -629,16 +677,18 @@ int hr_xtc_decode(const void* data, int64_t n_bytes, const int64_t* offsets, int
                "NULL pointer argument");
     HR_REQUIRE((reinterpret_cast<uintptr_t>(data) & 3) == 0, "data must be 4-byte aligned");
     HR_REQUIRE((reinterpret_cast<uintptr_t>(xyz) & 3) == 0, "xyz must be 4-byte aligned");
-    const int r = xtc_row_lanes(n_frames);
-    const auto kernel = r == 8    ? xtc_decode_kernel<8>
+    const bool tiny = n_atoms <= kTinyAtoms;
+    const int r = tiny ? kTinyLanes : xtc_row_lanes(n_frames);
+    const auto kernel = tiny      ? xtc_tiny_kernel
+                        : r == 8  ? xtc_decode_kernel<8>
                         : r == 16 ? xtc_decode_kernel<16>
                         : r == 32 ? xtc_decode_kernel<32>
                                   : xtc_decode_kernel<64>;
-    const long long waves = (n_frames + kWave / r - 1) / (kWave / r);
-    hipLaunchKernelGGL(kernel, launch_grid(waves, kWave), dim3(kWave), 0, (hipStream_t)stream,
-                       static_cast<const unsigned char*>(data), (long long)n_bytes,
-                       reinterpret_cast<const long long*>(offsets), (long long)n_frames, n_atoms,
-                       xyz, time, step, box, prec, status);
+    const int block = tiny ? kTinyBlock : kWave, frames = block / r;  // of a workgroup
+    hipLaunchKernelGGL(kernel, launch_grid((n_frames + frames - 1) / frames, block), dim3(block), 0,
+                       (hipStream_t)stream, static_cast<const unsigned char*>(data),
+                       (long long)n_bytes, reinterpret_cast<const long long*>(offsets),
+                       (long long)n_frames, n_atoms, xyz, time, step, box, prec, status);
     return launch_status("xtc_decode_kernel");
 }
 
