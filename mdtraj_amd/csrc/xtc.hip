@@ -15,7 +15,7 @@
 // small atoms as deltas (one mixed-radix number of smallidx bits each).
 //
 // Frames are independent, so the host walks the headers once (hr_xtc_scan,
-// the frame index) and the device decodes one frame per row of 8 to 64 lanes:
+// the frame index) and the device decodes one frame per row of 4 to 64 lanes:
 // where a group of atoms starts depends on the flags of all before it, but
 // once the starts are known the groups decode side by side.  Every read is bounded by the frame's
 // own bytes and every write by its atom count; a malformed frame ends with a
@@ -111,8 +111,8 @@ struct XtcRow {
 // spare, and so does the staging area.  A batch that finds too few words takes
 // no group but is followed by a refill, so the batches end.
 constexpr int kMaxGroupBits = 96 + 6 + 10 * 72;
-static_assert((XtcRow<8>::kRing - XtcRow<8>::kBlock4) * 32 >= kMaxGroupBits + 64, "ring");
-static_assert(XtcRow<8>::kCap >= 11, "staging area");
+static_assert((XtcRow<4>::kRing - XtcRow<4>::kBlock4) * 32 >= kMaxGroupBits + 64, "ring");
+static_assert(XtcRow<4>::kCap >= 11, "staging area");
 
 // Orders the wave's LDS accesses (the workgroup is one wave, whose LDS
 // accesses complete in program order; this keeps the compiler from moving
@@ -194,7 +194,7 @@ __device__ __forceinline__ void ring_ints3(const uint32_t* ring, uint32_t base, 
     out[1] = (uint32_t)r2;
 }
 
-// Lanes of a frame's row, by the number of frames: the narrowest row that
+// Lanes of a frame's row, by the number of frames: in general the narrowest row that
 // leaves the chip enough waves.  A step of the scan costs a wave the same
 // whatever its rows are, so narrow rows scan more frames for it, but a frame
 // alone is done sooner the wider its row (us, rows of 8 / 16 / 32 / 64 lanes):
@@ -207,7 +207,23 @@ __device__ __forceinline__ void ring_ints3(const uint32_t* ring, uint32_t base, 
 // 90,000 x 600              428 / 493 / 649 / 954
 // (one frame per lane, decoded in series: 1,590 us on 90,000 water frames of
 // 600 atoms, 3,254 us on 10,000 x 3,001).
-inline int xtc_row_lanes(long long n_frames) {
+//
+// A frame of a few dozen atoms has too few groups for eight lanes, and many such
+// frames leave a wave little to do (us with rows of 4 / 8 lanes, on streams whose
+// flags are rarely and always set; with one frame per lane, 500,000 x 12 atoms
+// took 181 and 146 us):
+//  16,000 x 12 atoms    11 / 10     11 / 10
+//  65,536 x 12          19 / 23     19 / 25
+//  65,536 x 20          29 / 32     22 / 29
+//  80,000 x 20          38 / 38     27 / 33
+//  80,000 x 22          41 / 39     29 / 35
+// 500,000 x 12          96 / 134    96 / 152
+// 500,000 x 22         167 / 187   118 / 171
+constexpr int kNarrowAtoms = 20;
+constexpr long long kNarrowFrames = 65536;
+
+inline int xtc_row_lanes(long long n_frames, int n_atoms) {
+    if (n_atoms <= kNarrowAtoms && n_frames >= kNarrowFrames) return 4;
     return n_frames >= 16000 ? 8 : n_frames >= 6000 ? 16 : n_frames >= 3000 ? 32 : 64;
 }
 
@@ -678,8 +694,9 @@ int hr_xtc_decode(const void* data, int64_t n_bytes, const int64_t* offsets, int
     HR_REQUIRE((reinterpret_cast<uintptr_t>(data) & 3) == 0, "data must be 4-byte aligned");
     HR_REQUIRE((reinterpret_cast<uintptr_t>(xyz) & 3) == 0, "xyz must be 4-byte aligned");
     const bool tiny = n_atoms <= kTinyAtoms;
-    const int r = tiny ? kTinyLanes : xtc_row_lanes(n_frames);
+    const int r = tiny ? kTinyLanes : xtc_row_lanes(n_frames, n_atoms);
     const auto kernel = tiny      ? xtc_tiny_kernel
+                        : r == 4  ? xtc_decode_kernel<4>
                         : r == 8  ? xtc_decode_kernel<8>
                         : r == 16 ? xtc_decode_kernel<16>
                         : r == 32 ? xtc_decode_kernel<32>
