@@ -811,6 +811,7 @@ __global__ __launch_bounds__(kBlock) void centroid_kernel(const float* __restric
 // of |d|^2 in FP64, so E|d|^2 - |E d|^2 does not cancel far from the origin.
 // Bound by HBM: 480 MB (20,000 frames of 2,000 atoms, every line of a 75 %
 // selection) in 99 us, 4.85 TB/s.
+template <int kEach>
 __global__ __launch_bounds__(kBlock) void rmsf_accum_kernel(
     const float* __restrict__ xyz, long long n_frames, int n_atoms, const int* __restrict__ idx,
     int n_sel, const float* __restrict__ rot, const double* __restrict__ mu, int n_chunks,
@@ -845,7 +846,6 @@ __global__ __launch_bounds__(kBlock) void rmsf_accum_kernel(
     double sx = 0.0, sy = 0.0, sz = 0.0, ss = 0.0;
     // the loads of kEach frames are in flight together (the chunk's last frame
     // again past its end)
-    constexpr int kEach = 8;
     const long long stride = 3LL * n_atoms;
     for (long long f = f0; f < f1; f += kEach) {
         float ax[kEach], ay[kEach], az[kEach];
@@ -921,6 +921,28 @@ __global__ __launch_bounds__(kFinishWaves * kWave) void rmsf_finish_kernel(
         const double msf = mean - m2;
         out[j] = (float)sqrt(msf > 0.0 ? msf : 0.0);
     }
+}
+
+// The same for up to kFewChunks chunks (few frames or very many atoms), a
+// thread per atom: 16 waves with at most one chunk each are mostly launches
+// (us a call with 16 waves / a thread per atom: 3 frames of 50,000 atoms without
+// a fit 13.9 / 10.2, with one 508 / 454; 10 frames of 10,000 118 / 116; 50 of
+// 50,000 803 / 806.  With 20 chunks, 20 frames of 3,000 atoms: 49 / 51).
+constexpr int kFewChunks = 16;
+
+__global__ __launch_bounds__(kBlock) void rmsf_finish_few_kernel(
+    const double* __restrict__ partial, int n_chunks, int n_sel, long long n_frames,
+    float* __restrict__ out) {
+    const int j = blockIdx.x * kBlock + threadIdx.x;
+    if (j >= n_sel) return;
+    double s[4] = {0.0, 0.0, 0.0, 0.0};
+    for (int c = 0; c < n_chunks; ++c) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s[e] += partial[((size_t)c * n_sel + j) * 4 + e];
+    }
+    const double n = (double)n_frames, mx = s[0] / n, my = s[1] / n, mz = s[2] / n;
+    const double msf = s[3] / n - (mx * mx + my * my + mz * mz);
+    out[j] = (float)sqrt(msf > 0.0 ? msf : 0.0);
 }
 
 // Frame chunks of the RMSF accumulation: about 2,048 workgroups in all (eight
@@ -1265,12 +1287,16 @@ int hr_rmsf(const float* xyz, int64_t n_frames, int32_t n_atoms, const int32_t* 
     }
     const int n_chunks = rmsf_chunks(n_frames, n_sel);
     const int atom_blocks = (n_sel + kBlock - 1) / kBlock;
-    hipLaunchKernelGGL(rmsf_accum_kernel, dim3(atom_blocks, n_chunks), dim3(kBlock), 0, s, xyz,
+    // chunks of one frame do no more than that frame
+    const auto accum = n_chunks < n_frames ? rmsf_accum_kernel<8> : rmsf_accum_kernel<1>;
+    hipLaunchKernelGGL(accum, dim3(atom_blocks, n_chunks), dim3(kBlock), 0, s, xyz,
                        (long long)n_frames, n_atoms, atom_idx, n_sel, ref_frame ? rot : nullptr,
                        center ? mu : nullptr, n_chunks, partial);
     if ((rc = launch_status("rmsf_accum_kernel"))) return rc;
-    hipLaunchKernelGGL(rmsf_finish_kernel, dim3((n_sel + kFinishAtoms - 1) / kFinishAtoms),
-                       dim3(kFinishWaves * kWave), 0, s, partial, n_chunks, n_sel,
+    const bool few = n_chunks <= kFewChunks;
+    hipLaunchKernelGGL(few ? rmsf_finish_few_kernel : rmsf_finish_kernel,
+                       dim3(few ? atom_blocks : (n_sel + kFinishAtoms - 1) / kFinishAtoms),
+                       dim3(few ? kBlock : kFinishWaves * kWave), 0, s, partial, n_chunks, n_sel,
                        (long long)n_frames, out);
     return launch_status("rmsf_finish_kernel");
 }
