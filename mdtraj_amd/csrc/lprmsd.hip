@@ -26,6 +26,8 @@
 // serial steps, about 119,000 cycles (gather 17, fit 16, nearest columns 41,
 // two searches of two passes 25, the rest 20 thousand) with eight frames
 // resident per CU.
+#include <type_traits>
+
 #include "common.h"
 
 namespace hr {
@@ -514,99 +516,113 @@ __global__ __launch_bounds__(kLpFrameBlock, 4) void lp_frame_kernel(LpArgs A) {
             way[j] = 0;
         }
         wave_sync();
-        for (int s = 0; s * kWave < k; ++s) {
-            for (unsigned long long rows = __ballot((free_rows >> s) & 1u); rows; rows &= rows - 1) {
-                const int i = s * kWave + __ffsll((long long)rows);
-                for (int j = lane; j <= k; j += kWave) {
-                    minv[j] = __builtin_huge_val();
-                    used[j] = 0;
-                }
-                if (lane == 0) p[0] = i;
-                wave_sync();
-                int j0 = 0;
-                // each pass marks one more column used; a free column (p = 0) is
-                // reached within i passes, so the loop ends for any costs
-                for (int pass = 0; pass <= k; ++pass) {
-                    if (lane == 0) used[j0] = 1;
+        // The rows left over, kEach columns a lane at a time: as many as a group
+        // has for each lane up to five, so that a group of a few atoms does not
+        // handle five strips of columns for its one; two for groups of more than
+        // five strips, where a last batch of five would be mostly repeats (us a
+        // call of five for all / this, diffused: see below).
+        auto search = [&](auto each) {
+            constexpr int kEach = decltype(each)::value;
+            for (int s = 0; s * kWave < k; ++s) {
+                for (unsigned long long rows = __ballot((free_rows >> s) & 1u); rows; rows &= rows - 1) {
+                    const int i = s * kWave + __ffsll((long long)rows);
+                    for (int j = lane; j <= k; j += kWave) {
+                        minv[j] = __builtin_huge_val();
+                        used[j] = 0;
+                    }
+                    if (lane == 0) p[0] = i;
                     wave_sync();
-                    const int i0 = p[j0];
-                    const float qx = grx[i0 - 1], qy = gry[i0 - 1], qz = grz[i0 - 1];
-                    const double ui = u[i0];
-                    double best = __builtin_huge_val();
-                    int at = INT_MAX;
-                    for (int b0 = 1 + lane; b0 <= k; b0 += kLpBatch * kWave) {
-                        bool open[kLpBatch];
-                        int ta[kLpBatch];
-                        double vj[kLpBatch], mv[kLpBatch];
-                        float dx[kLpBatch], dy[kLpBatch], dz[kLpBatch];
-#pragma unroll
-                        for (int t = 0; t < kLpBatch; ++t) {
-                            const int j = min(b0 + t * kWave, k);
-                            open[t] = b0 + t * kWave <= k && !used[j];
-                            ta[t] = gat[j - 1];
-                            vj[t] = v[j];
-                            mv[t] = minv[j];
-                        }
-#pragma unroll
-                        for (int t = 0; t < kLpBatch; ++t) {
-                            dx[t] = qx - tx[ta[t]];
-                            dy[t] = qy - ty[ta[t]];
-                            dz[t] = qz - tz[ta[t]];
-                        }
-#pragma unroll
-                        for (int t = 0; t < kLpBatch; ++t) {
-                            const int j = b0 + t * kWave;
-                            const double cur = lp_cost(dx[t], dy[t], dz[t]) - ui - vj[t];
-                            if (open[t]) {
-                                if (cur < mv[t]) {
-                                    mv[t] = cur;
-                                    minv[j] = cur;
-                                    way[j] = j0;
-                                }
-                                if (mv[t] < best || at == INT_MAX) {
-                                    best = mv[t];
-                                    at = j;
+                    int j0 = 0;
+                    // each pass marks one more column used; a free column (p = 0) is
+                    // reached within i passes, so the loop ends for any costs
+                    for (int pass = 0; pass <= k; ++pass) {
+                        if (lane == 0) used[j0] = 1;
+                        wave_sync();
+                        const int i0 = p[j0];
+                        const float qx = grx[i0 - 1], qy = gry[i0 - 1], qz = grz[i0 - 1];
+                        const double ui = u[i0];
+                        double best = __builtin_huge_val();
+                        int at = INT_MAX;
+                        for (int b0 = 1 + lane; b0 <= k; b0 += kEach * kWave) {
+                            bool open[kEach];
+                            int ta[kEach];
+                            double vj[kEach], mv[kEach];
+                            float dx[kEach], dy[kEach], dz[kEach];
+    #pragma unroll
+                            for (int t = 0; t < kEach; ++t) {
+                                const int j = min(b0 + t * kWave, k);
+                                open[t] = b0 + t * kWave <= k && !used[j];
+                                ta[t] = gat[j - 1];
+                                vj[t] = v[j];
+                                mv[t] = minv[j];
+                            }
+    #pragma unroll
+                            for (int t = 0; t < kEach; ++t) {
+                                dx[t] = qx - tx[ta[t]];
+                                dy[t] = qy - ty[ta[t]];
+                                dz[t] = qz - tz[ta[t]];
+                            }
+    #pragma unroll
+                            for (int t = 0; t < kEach; ++t) {
+                                const int j = b0 + t * kWave;
+                                const double cur = lp_cost(dx[t], dy[t], dz[t]) - ui - vj[t];
+                                if (open[t]) {
+                                    if (cur < mv[t]) {
+                                        mv[t] = cur;
+                                        minv[j] = cur;
+                                        way[j] = j0;
+                                    }
+                                    if (mv[t] < best || at == INT_MAX) {
+                                        best = mv[t];
+                                        at = j;
+                                    }
                                 }
                             }
                         }
-                    }
-                    wave_argmin(best, at);
-                    const double delta = best;
-                    wave_sync();  // every lane has read u[i0] before it changes
-                    for (int b0 = lane; b0 <= k; b0 += kLpBatch * kWave) {
-                        bool taken[kLpBatch];
-                        double was[kLpBatch];
-#pragma unroll
-                        for (int t = 0; t < kLpBatch; ++t) taken[t] = used[min(b0 + t * kWave, k)];
-#pragma unroll
-                        for (int t = 0; t < kLpBatch; ++t) {
-                            const int j = min(b0 + t * kWave, k);
-                            was[t] = taken[t] ? v[j] : minv[j];
-                        }
-#pragma unroll
-                        for (int t = 0; t < kLpBatch; ++t) {
-                            const int j = b0 + t * kWave;
-                            if (j <= k) {
-                                if (taken[t]) u[p[j]] += delta;
-                                (taken[t] ? v : minv)[j] = was[t] - delta;
+                        wave_argmin(best, at);
+                        const double delta = best;
+                        wave_sync();  // every lane has read u[i0] before it changes
+                        for (int b0 = lane; b0 <= k; b0 += kEach * kWave) {
+                            bool taken[kEach];
+                            double was[kEach];
+    #pragma unroll
+                            for (int t = 0; t < kEach; ++t) taken[t] = used[min(b0 + t * kWave, k)];
+    #pragma unroll
+                            for (int t = 0; t < kEach; ++t) {
+                                const int j = min(b0 + t * kWave, k);
+                                was[t] = taken[t] ? v[j] : minv[j];
                             }
+    #pragma unroll
+                            for (int t = 0; t < kEach; ++t) {
+                                const int j = b0 + t * kWave;
+                                if (j <= k) {
+                                    if (taken[t]) u[p[j]] += delta;
+                                    (taken[t] ? v : minv)[j] = was[t] - delta;
+                                }
+                            }
+                        }
+                        wave_sync();
+                        j0 = at;
+                        if (p[j0] == 0) break;
+                    }
+                    if (lane == 0) {
+                        int jj = j0;
+                        for (int step = 0; step <= k && jj != 0; ++step) {
+                            const int j1 = way[jj];
+                            p[jj] = p[j1];
+                            jj = j1;
                         }
                     }
                     wave_sync();
-                    j0 = at;
-                    if (p[j0] == 0) break;
                 }
-                if (lane == 0) {
-                    int jj = j0;
-                    for (int step = 0; step <= k && jj != 0; ++step) {
-                        const int j1 = way[jj];
-                        p[jj] = p[j1];
-                        jj = j1;
-                    }
-                }
-                wave_sync();
             }
-        }
+        };
+        if (k < kWave)
+            search(std::integral_constant<int, 1>{});
+        else if (k < 2 * kWave || k >= kLpBatch * kWave)
+            search(std::integral_constant<int, 2>{});
+        else
+            search(std::integral_constant<int, kLpBatch>{});
         // column j (target atom gat[j - 1]) takes row p[j] (reference atom gat[p[j] - 1])
         for (int j = 1 + lane; j <= k; j += kWave) {
             const int ta = gat[j - 1], ra = p[j] - 1;
