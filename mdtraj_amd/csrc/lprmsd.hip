@@ -446,8 +446,30 @@ __global__ __launch_bounds__(kLpFrameBlock, 4) void lp_frame_kernel(LpArgs A) {
             if (lead && lane == 0) A.out[f] = __builtin_nanf("");
             return;
         }
+        if (k == 1) {  // one atom keeps its label (100 such groups: 1,600 us a call, now 240)
+            if (threadIdx.x == 0) {
+                const int a = clamp_index(A.group_atoms[g0], n);
+                const double t[3] = {tx[a], ty[a], tz[a]};
+                const double r[3] = {rx[a], ry[a], rz[a]};
+#pragma unroll
+                for (int i = 0; i < 3; ++i)
+#pragma unroll
+                    for (int j = 0; j < 3; ++j) M2[3 * i + j] = fma(t[i], r[j], M2[3 * i + j]);
+            }
+            continue;
+        }
+        // The second wave's rows start at the 33rd: smaller groups are the first
+        // wave's alone, without workgroup barriers (10,000 frames of 50 groups of
+        // two: 827 us with them, 626 without; diffused 1,120 / 826).
+        if (!lead && k <= kWave / 2) continue;
         float* q = reinterpret_cast<float*>(minv);
         int* col = reinterpret_cast<int*>(v);
+        auto sync = [&] {  // of the waves that share the group
+            if (k > kWave / 2)
+                __syncthreads();
+            else
+                wave_sync();
+        };
         // the group's target atoms where minv, p and way will be (16 k1 bytes,
         // after two arrays of 8 k1), the rows' columns where v will be
         if (lead) {
@@ -485,19 +507,20 @@ __global__ __launch_bounds__(kLpFrameBlock, 4) void lp_frame_kernel(LpArgs A) {
                 s_biggest = biggest;
             }
         }
-        __syncthreads();
+        sync();
         // Greedy start: every row's least cost as its dual, and the row itself
         // in that column unless a lower row is there.  Rows left over (two
         // reference atoms nearest to one target atom) are searched for; from
         // empty duals every row was (8.0 ms a call of 20,000 frames x 300
         // interchangeable atoms).
-        if (!lp_row_minima(q, k, grx, gry, grz, s_biggest, u, col, lane, lead ? 0 : 32)) s_finite = 0;
-        __syncthreads();
+        if (!lp_row_minima(q, k, grx, gry, grz, s_biggest, u, col, lane, lead ? 0 : 32))
+            s_finite = 0;
+        sync();
         if (!lead) continue;
         const bool greedy = s_finite != 0;
         for (int j = lane; j <= k; j += kWave) {
             p[j] = greedy ? INT_MAX : 0;
-            way[j] = j ? col[j] : 0;
+            way[j] = j && greedy ? col[j] : 0;
             if (!greedy || j == 0) u[j] = 0.0;
         }
         wave_sync();
@@ -516,11 +539,11 @@ __global__ __launch_bounds__(kLpFrameBlock, 4) void lp_frame_kernel(LpArgs A) {
             way[j] = 0;
         }
         wave_sync();
-        // The rows left over, kEach columns a lane at a time: as many as a group
-        // has for each lane up to five, so that a group of a few atoms does not
-        // handle five strips of columns for its one; two for groups of more than
-        // five strips, where a last batch of five would be mostly repeats (us a
-        // call of five for all / this, diffused: see below).
+        // The rows left over, kEach columns a lane at a time: one or two where the
+        // group has no more, five for up to five, two beyond, where a last five
+        // would be mostly repeats.  Us a call of diffused atoms with five always /
+        // so: 10,000 frames of 100 atoms 5,300 / 4,000, of 32 atoms 807 / 467, one
+        // frame of 100 atoms 1,020 / 780, 500 of 700 102,000 / 93,000.
         auto search = [&](auto each) {
             constexpr int kEach = decltype(each)::value;
             for (int s = 0; s * kWave < k; ++s) {

@@ -46,6 +46,31 @@ def test_groups_without_atoms(gpu, groups):
     assert np.abs(y - moved).max() < 2e-5
 
 
+@pytest.mark.parametrize("sizes", [(1,), (1, 1, 1), (2, 1, 2), (31, 1), (32, 33, 32), (33, 1, 2, 64),
+                                   (129, 2, 192), (200, 1), (256,), (320, 40), (385,)])
+@pytest.mark.parametrize("noise", [0.02, 0.5])
+def test_several_groups(gpu, sizes, noise):
+    """Groups of one wave beside groups of both, single atoms beside them, and
+    searches of one, two and five columns a lane at a time, with superposition."""
+    rng = np.random.default_rng(sum(sizes))
+    n = 9 + sum(sizes)
+    base = np.concatenate([rng.normal(0, 0.6, (9, 3)), rng.uniform(-1, 1, (n - 9, 3))])
+    x = base[None] + rng.normal(0, noise, (3, n, 3))
+    groups, at = [], 9
+    for k in sizes:
+        groups.append(np.arange(at, at + k))
+        for f in range(3):
+            x[f, at:at + k] = x[f, at + rng.permutation(k)]
+        at += k
+    x = x.astype(np.float32)
+    ref = base[None].astype(np.float32)
+    want, moved = olp.lprmsd(x, ref, 0, None, groups, superpose=True)
+    y = x.copy()
+    got = md.lprmsd(y, ref, 0, permute_groups=groups, superpose=True)
+    assert np.abs(got - want).max() < 2e-5
+    assert np.abs(y - moved).max() < 2e-5
+
+
 def test_more_frames_than_one_launch_dimension(gpu):
     """2^25 + 3 frames of two waves each: above 2^32 work-items.  The frames
     repeat, so every result is one of a few."""
