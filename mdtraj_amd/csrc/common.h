@@ -61,21 +61,25 @@ inline int launch_status(const char* what) {
     return HR_OK;
 }
 
-// Grid of a kernel that has one workgroup per `groups`, as rows of equal length
-// short enough for a launch: from 2^32 work-items in one dimension on (33.5 M
-// workgroups of 128) the count wraps, and what is past it is left out without an
-// error.  workgroup_index() numbers the workgroups; the last may lie past `groups`.
+// Grid of a kernel that has one workgroup per `groups` (up to 2^32 - 2^16 of them):
+// one row of them, or rows of 2^16 where a row would reach 2^32 work-items (33.5 M
+// workgroups of 128), from where on the count in a launch's dimension wraps and
+// what is past it is left out without an error.  workgroup_index() numbers the
+// workgroups, without a load of the grid's size (which cost the lane-per-frame
+// kernel 0.6 %); the last ones may lie past `groups`.
+constexpr int kGridRowLog2 = 16;
+
 inline dim3 launch_grid(long long groups, int threads) {
-    const long long most = 0xFFFFFFFFLL / threads;
-    const long long rows = (groups + most - 1) / most;
-    return dim3((unsigned)((groups + rows - 1) / rows), (unsigned)rows);
+    if (groups <= 0xFFFFFFFFLL / threads) return dim3((unsigned)groups);
+    return dim3(1u << kGridRowLog2,
+                (unsigned)((groups + (1 << kGridRowLog2) - 1) >> kGridRowLog2));
 }
 
 // --------------------------------------------------------------- device side
 constexpr int kWave = 64;
 
 __device__ __forceinline__ long long workgroup_index() {
-    return (long long)blockIdx.y * gridDim.x + blockIdx.x;
+    return ((long long)blockIdx.y << kGridRowLog2) + blockIdx.x;
 }
 
 // Coordinates, references and indices always live in global memory, but a

@@ -38,10 +38,12 @@ def grid():
 
 @pytest.mark.parametrize("threads", [64, 128, 256])
 @pytest.mark.parametrize("groups", [1, 2, 1000003, 2**24 - 1, 2**24, 2**25 - 1, 2**25, 2**25 + 1,
-                                    2**26, 2**31 - 1, 2**31, 2**32 + 7, 2**36])
+                                    2**26, 2**31 - 1, 2**31, 2**32 - 2**16])
 def test_every_workgroup_within_the_launch_limits(grid, groups, threads):
     x, y, z = grid(groups, threads)
     assert z == 1 and x * threads < 2**32 and x < 2**31 and y < 2**16
-    assert groups <= x * y < groups + y  # at most one row's remainder past the end
+    assert groups <= x * y < groups + 2**16  # at most one row's remainder past the end
     if groups * threads < 2**32:
-        assert y == 1
+        assert (x, y) == (groups, 1)
+    else:
+        assert x == 2**16  # what workgroup_index() counts a row as
