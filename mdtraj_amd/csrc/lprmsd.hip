@@ -275,11 +275,11 @@ __device__ __forceinline__ bool lp_row_minima(const float* q, int k, const float
         const bool mine = half == 0 && r0 + in < k;
         const float* near = q + 4 * min(args[0], k - 1);
         double least = lp_cost(x - near[0], y - near[2], z - near[1]);
-        const float m = fmaxf(aa, biggest), tol = 0x1p-15f * m;
-        const bool plain = m > 0x1p-96f && m < 0x1p96f;
+        const float m = fmaxf(aa, biggest);
+        const float tol = m > 0x1p-96f && m < 0x1p96f ? 0x1p-15f * m : __builtin_huge_valf();
         // the close rows, one by one, the columns spread over the lanes
-        for (unsigned long long close = __ballot(mine && !(plain && second[0] > best[0] + tol));
-             close; close &= close - 1) {
+        for (unsigned long long close = __ballot(mine && !(second[0] > best[0] + tol)); close;
+             close &= close - 1) {
             const int l = __ffsll((long long)close) - 1;
             const float rx = __shfl(x, l, kWave), ry = __shfl(y, l, kWave), rz = __shfl(z, l, kWave);
             double c_best = __builtin_huge_val();
