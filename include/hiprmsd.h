@@ -50,6 +50,10 @@ int hr_device_cu_count(void);
 
 /* Tuning knobs (no counterpart in the reference; set by the autotuner in
  * mdtraj_amd/autotune.py).  Values are process-wide; 0 restores the default.
+ * The per-frame kernel's knobs (HR_TUNE_FRAMES_*) do not reach the calls that
+ * have a kernel of their own: one-vs-all RMSDs over whole frames of up to 40
+ * atoms (no atom_idx) and hr_superpose in one pass (see
+ * HR_TUNE_SUPERPOSE_CHUNK_MIB).
  *   HR_TUNE_FRAMES_WAVES_PER_SIMD  register budget of the per-frame kernel:
  *                                  3 (default, no spills) or 4 waves/SIMD
  *   HR_TUNE_FRAMES_GRID            accepted for compatibility (0, 1, 2);
@@ -76,13 +80,17 @@ int hr_device_cu_count(void);
  *                                  ~13,600 reference atoms in LDS) whose
  *                                  waves share each system's frames through
  *                                  an LDS counter
- *   HR_TUNE_SUPERPOSE_CHUNK_MIB    hr_superpose fits and rotates the frames
- *                                  in chunks of about this many MiB of
- *                                  coordinates (a fit pass, then a rotation
- *                                  pass, per chunk); 0 the default (1024), a
- *                                  value at least the trajectory's size one
- *                                  fit pass and one rotation pass over all
- *                                  frames.  Results do not depend on it.
+ *   HR_TUNE_SUPERPOSE_CHUNK_MIB    hr_superpose with align_xyz, or over
+ *                                  frames of which two do not fit a CU's LDS
+ *                                  (above about 6,600 atoms), fits and
+ *                                  rotates the frames in chunks of about
+ *                                  this many MiB of coordinates (a fit pass,
+ *                                  then a rotation pass, per chunk); 0 the
+ *                                  default (1024), a value at least the
+ *                                  trajectory's size one fit pass and one
+ *                                  rotation pass over all frames.  Results
+ *                                  do not depend on it.  All other calls
+ *                                  fit and rotate in one pass and ignore it.
  *   HR_TUNE_HOST_DIRECT_KIB        hr_rmsd_one_vs_all_host: selections of up
  *                                  to this many KiB in all (0: the default,
  *                                  1024) are read by the kernels straight

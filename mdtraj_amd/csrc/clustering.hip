@@ -145,8 +145,13 @@ __device__ __forceinline__ double rows8_sum(const double (&a)[8], int lane) {
 // Rows of a tile, which has 256 columns: few enough that the tiles fill the
 // chip.  Us of hr_centroid_scores with tiles of 256 rows, as many as columns,
 // and with these: 1,000 frames 78 / 27, 4,001 84 / 59, 8,000 174 / 154, 12,000
-// 274 / 202, 16,100 464 / 346.  32 and 64 rows are even at 8,000 frames; beyond,
-// the fewer column partials are the better.
+// 274 / 202, 16,100 464 / 346, 16,200 470 / 435.  32 and 64 rows are even at 8,000
+// frames; beyond, the fewer column partials are the better.
+// Columns of tiles in eights are slow for their size, 32 and 64 most (us just
+// below / in / just above: 24 columns 74 / 87 / 80, 32 110 / 154 / 113, 48 204 / 238 /
+// 215, 64 345 / 440 / 365): workgroups go to the eight XCDs in turn, and at 32 and 64
+// to the CUs too, so each gets tiles of the same columns in every row, and the
+// columns on the right have more of them.
 constexpr int kTallTile = 64, kLowTile = 32;
 constexpr long long kLowTileFrames = 8064;
 

@@ -17,7 +17,7 @@
 // Two waves per frame.  Most rows of a group need no search: every row's
 // nearest column is found first, on the matrix cores and by both waves, and
 // rows whose nearest columns differ are matched at once.  The first wave does
-// all else; the columns of a search are spread over its lanes, and the
+// all else (and groups of up to 32 atoms alone); the columns of a search are spread over its lanes, and the
 // search's minimum is a wave reduction (ties to the lowest column).  The
 // group's reference coordinates, potentials and search state sit in LDS (sized
 // to keep eight frames per CU for groups of a few hundred atoms).
@@ -25,7 +25,11 @@
 // when every row was searched for, 0.60 ms now): the latency of a frame's
 // serial steps, about 119,000 cycles (gather 17, fit 16, nearest columns 41,
 // two searches of two passes 25, the rest 20 thousand) with eight frames
-// resident per CU.
+// resident per CU.  That is with atoms near their reference places; what a
+// diffused liquid costs is the searches themselves, which the start hardly
+// shortens (4,000 frames x (100 + 300), every row searched for / now: 0.02 nm of
+// noise 1.63 / 0.12 ms, 0.1 nm 2.05 / 0.66, 0.2 nm 12.7 / 10.1, independent places
+// 26.3 / 23.7).
 #include <type_traits>
 
 #include "common.h"

@@ -968,12 +968,15 @@ size_t rmsf_partials(long long n_frames, int n_sel) {
     return std::min(chunks * n_sel, (size_t)kRmsfGroups * kBlock + n_sel);
 }
 
-// Default chunk of hr_superpose (MiB of coordinates); HR_TUNE_SUPERPOSE_CHUNK_MIB
-// overrides it.  On 100,000 frames x 2,000 atoms (2.4 GB), chunks of 1 GiB
-// took 1.428 ms per call against 1.475 ms for one pass of each kernel;
-// chunks of 256 MiB or less are slower (each chunk pays the two kernels'
-// ramp and drain), so the rotation pass gains nothing measurable from
-// re-reading a chunk that is still cached.
+// Default chunk of hr_superpose's two kernels (MiB of coordinates);
+// HR_TUNE_SUPERPOSE_CHUNK_MIB overrides it.  They serve frames too long for one
+// pass and separate alignment arrays.  Us a call with chunks of 256 MiB / 1 GiB /
+// all frames at once: 25,000 frames x 8,000 atoms (2.4 GB) 2,017 / 1,803 / 1,670,
+// 8,000 x 25,000 3,194 / 2,097 / 1,751, 10,000 x 8,000 with an alignment array
+// 1,078 / 733 / 734, 100,000 x 2,000 with one 1,543 / 1,398 / 1,365: each chunk pays
+// the two kernels' ramp and drain, and the rotation gains nothing from a chunk
+// that is still cached.  (1 GiB was the better by 3 % where all frames of 2,000
+// atoms took this path; at the sizes that are left one chunk would be.)
 constexpr int kSuperposeChunkMiB = 1024;
 
 }  // namespace

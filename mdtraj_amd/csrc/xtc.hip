@@ -205,8 +205,11 @@ __device__ __forceinline__ void ring_ints3(const uint32_t* ring, uint32_t base, 
 // 16,000 x 1,000            167 / 166 / 207 / 295
 // 60,000 x 43                49 / 70 / 107 / 181
 // 90,000 x 600              428 / 493 / 649 / 954
-// (one frame per lane, decoded in series: 1,590 us on 90,000 water frames of
-// 600 atoms, 3,254 us on 10,000 x 3,001).
+// (one frame per lane, decoded in series: 3,254 us on 10,000 x 3,001).  These are
+// streams of a chain in water with long runs, 0.3 groups an atom.  The water
+// file that the tests read, written by the reference's encoder, has 0.93 groups
+// an atom: 90,000 of its frames (600 atoms) take 789 us in rows of 8, 1,590 with
+// one frame per lane.
 //
 // A frame of a few dozen atoms has too few groups for eight lanes, and many such
 // frames leave a wave little to do (us with rows of 4 / 8 lanes, on streams whose
