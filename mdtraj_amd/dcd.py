@@ -42,7 +42,7 @@ def cell_lengths_angles(cell):
     # a constant cell: one row's angles serve all (10,001 frames 666 -> 175 us; below
     # 512 the comparison costs more than the angles).  A changing cell, which
     # differs in its last frame too, does not pay for comparing every row.
-    if n >= 512 and (c[-1] == c[0]).all() and (c == c[0]).all():
+    if n >= 512 and c[-1].tolist() == c[0].tolist() and (c == c[0]).all():
         lengths, angles = cell_lengths_angles(c[:1])
         return np.repeat(lengths, n, axis=0), np.repeat(angles, n, axis=0)
     lengths = c[:, [0, 2, 5]].copy()
